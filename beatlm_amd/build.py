@@ -38,6 +38,7 @@ SOURCES = [
     "k_gemm_f32.hip",
     "k_gemm_split.hip",
     "k_gemm_f16.hip",
+    "k_wave.hip",
     "k_flash.hip",
     "k_misc.hip",
     "static_attention.hip",

@@ -679,7 +679,7 @@ void keep_split_activations(bl_kernels *ks, const bl_spec *specs, uint32_t n, co
                 const Launch &L = ks->kernels[ki].per_set[si];
                 const GemmArgs &g = L.gemm;
                 ok = L.family == Family::GEMM && L.math == Math::SPLIT && L.gemm.pipeline &&
-                     (conv ? g.load == 3 && gemm_tile_cols(L.tile) >= 64 && g.p2 % 32 == 0 &&
+                     (conv ? g.load == 3 && (gemm_tile_cols(L.tile) >= 64 || gemm_tile_wave(L.tile)) && g.p2 % 32 == 0 &&
                                  (uint64_t)(g.p0 + 1) * (g.p1 + 1) * g.p2 < (1ull << 31) && 9ull * g.p2 < (1u << 16) &&
                                  !getenv("BL_CONV_NO_SPLIT_INPUT")
                           : g.load == 0 && g.k % 32 == 0);
@@ -963,6 +963,106 @@ void plan_folds(bl_kernels *ks, const bl_spec *specs, uint32_t n, const bl_bindi
     }
     ks->fold_state.valid.assign(ks->folds.size() * n_sets, 0);
     ks->fold_state.touched.assign(ks->folds.size() * n_sets, 0);
+}
+
+// The wave-split kernel's tile for a product, or -1 for the ring kernel: the
+// smallest of 16 x 32, 32 x 32 and 32 x 64 whose tiles all run at once (a
+// workgroup per CU). In one round the smaller tile is the shorter chain of
+// loads; a second round doubles the launch (us, one process, ring / 16 x 32 /
+// 32 x 32 / 32 x 64; bf16x3 unless said):
+//   fc2 1536 -> 384,  257 tokens: 12.3 /  6.2 /  7.0 /  8.9  (204, 108, 54 tiles)
+//                     362 tokens: 12.3 / 10.6 /  7.0 /  9.1  (276, 144, 72)
+//                    1025 tokens: 12.9 / 19.5 / 13.1 /  9.4  (780, 396, 198)
+//                    1370 tokens: 13.8 / 24.8 / 18.8 / 18.3  (1032, 516, 258: the ring)
+//   fc2 3072 -> 768 f16, 626 tokens: 24.9 / 26.6 / 15.9 / 11.4
+//   fc2 1536 -> 384 on the f32 matrix cores, 626 tokens: 39.9 / 16.8 / 13.4 / 21.4
+//   convolution 64 -> 64 over 19 x 19 (split k and its reduce / ...): 8.3 / 5.9 / 7.6 / 8.7;
+//                            over 74 x 74: 15.2 / 12.0 / 14.3 / 9.5
+//   patch embedding 588 -> 384, 169 patches: 16.9 / 5.8 / 7.6 / 10.7
+// Weights beyond an XCD's L2 (6 MB: 4096 -> 1024) come from further away for
+// every row of tiles: 32 rows at least (f16, 65 tokens: 17.9 / 9.2 / 7.1). A
+// product of one 64-wide step takes the 32 x 64 ring tile rather than the
+// same tile here (74 x 74 x 64 -> 64: 4.1 against 4.5). The f32 matrix cores
+// are slow enough that long products want more workgroups than one per
+// tile: convolutions of more than 2048 keep split k (384 -> 64 over 13 x 13:
+// 12.3 against 15.1), and the 32 x 64 tile is only for products longer than
+// 512 (QKV at 257 tokens: 8.2 against 8.5). BL_GEMM_WAVE: 0 none, 1 .. 3 that
+// tile wherever the kernel takes the product.
+int wave_tile_of(const GemmArgs &g, Math m, uint32_t compute_units, int mode) {
+    const int tiles[] = {TILE_W16x32, TILE_W32x32, TILE_W32x64};
+    if (mode >= 1 && mode <= 3) return tiles[mode - 1];
+    const uint64_t weight_bytes = (uint64_t)g.n * g.k * (m == Math::F16 ? 2 : 4);
+    if (m == Math::F32 && g.load == 3 && g.k > 2048) return -1;
+    for (int t : tiles) {
+        if (t == TILE_W16x32 && weight_bytes > (6u << 20) && g.row1 - g.row0 > 16) continue;
+        if (t == TILE_W32x64 && (g.k <= 64 || (m == Math::F32 && g.k <= 512))) continue;
+        const uint64_t rows = (g.row1 - g.row0 + gemm_tile_rows(t) - 1) / gemm_tile_rows(t);
+        if (rows * ((g.n + gemm_tile_cols(t) - 1) / gemm_tile_cols(t)) <= compute_units) return t;
+    }
+    return -1;
+}
+
+// Gives products to the wave-split kernel (k_wave.hip) where wave_tile_of says
+// so, in every binding set, in place of a ring or of a split k and its reduce
+// launch. Not a projection that writes a flash kernel's operands, nor the
+// consumer of a folded LayerNorm.
+void plan_waves(bl_kernels *ks, uint32_t compute_units) {
+    const char *knob = getenv("BL_GEMM_WAVE");
+    const int mode = knob ? atoi(knob) : -1;
+    if (mode == 0) return;
+    // The knobs of the ring kernel ask for the ring kernel.
+    if (mode < 0)
+        for (const char *ring : {"BL_GEMM_TILE", "BL_GEMM_KGROUPS", "BL_GEMM_STAGES", "BL_GEMM_KSLICES", "BL_GEMM_BREG",
+                                 "BL_GEMM_LANE_EPILOGUE", "BL_CONV_SPLIT_K", "BL_CONV_NO_SPLIT_K"})
+            if (getenv(ring)) return;
+    std::vector<int> tiles(ks->kernels.size(), -1);
+    for (size_t ki = 0; ki < ks->kernels.size(); ki++) {
+        const Kernel &k = ks->kernels[ki];
+        int &tile = tiles[ki];
+        for (uint32_t si = 0; si < ks->sets; si++) {
+            const Launch &L = k.per_set[si];
+            int t = -1;
+            GemmArgs g = L.gemm;
+            g.ksplit = 1;
+            if (L.family == Family::GEMM && g.pipeline && L.tile != TILE_CONV3 && L.fold_role != FOLD_CONSUMER && gemm_wave_fits(g, L.math))
+                t = wave_tile_of(g, L.math, compute_units, mode);
+            // A projection of a flash kernel that takes its operands from it.
+            for (const Kernel &o : ks->kernels)
+                if (o.per_set[si].family == Family::FLASH && o.per_set[si].math != Math::F32 && o.per_set[si].fl.qkv == g.c) t = -1;
+            if (si == 0) tile = t;
+            else if (t != tile) tile = -1;
+        }
+    }
+    // A pack is fragment-major for all its readers or for none (a weight read
+    // by parts of different sizes, say).
+    std::vector<uint8_t> ring(ks->packs.size(), 0);
+    for (size_t ki = 0; ki < ks->kernels.size(); ki++)
+        for (const Launch &L : ks->kernels[ki].per_set)
+            if (L.pack >= 0 && tiles[ki] < 0) ring[L.pack] = 1;
+    for (bool again = true; again;) {
+        again = false;
+        for (size_t ki = 0; ki < ks->kernels.size(); ki++)
+            for (const Launch &L : ks->kernels[ki].per_set)
+                if (tiles[ki] >= 0 && ring[L.pack]) {
+                    tiles[ki] = -1;
+                    again = true;
+                    for (const Launch &o : ks->kernels[ki].per_set) ring[o.pack] = 1;
+                }
+    }
+    for (size_t ki = 0; ki < ks->kernels.size(); ki++) {
+        Kernel &k = ks->kernels[ki];
+        const int tile = tiles[ki];
+        if (tile < 0) continue;
+        for (Launch &L : k.per_set) {
+            L.tile = tile;
+            L.gemm.ksplit = L.gemm.kgroups = L.gemm.kslices = 1;
+        }
+        const Launch &L = k.per_set[0];
+        const size_t at = k.label.find(" @ "), end = k.label.find(" <", at), end2 = k.label.find(" >", at);
+        const std::string variant = std::string(" @ ") + (L.math == Math::F16 ? "mfma-f16" : L.math == Math::F32 ? "mfma-f32" : "mfma-bf16x3") +
+                                    " wave " + std::to_string(gemm_tile_rows(tile)) + "x" + std::to_string(gemm_tile_cols(tile));
+        k.label.replace(at, std::min(std::min(end, end2), k.label.size()) - at, variant);
+    }
 }
 
 // Bytes of a fold's buffers for one binding set: the statistics, then (f32
@@ -1388,7 +1488,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                     // "t" for every product, "t@n" for the products n columns wide.
                     const int t = atoi(force);
                     const char *at = strchr(force, '@');
-                    if (t >= 0 && t < TILE_COUNT && (!at || (uint32_t)atoi(at + 1) == gn)) {
+                    if (t >= 0 && t <= TILE_CONV3 && (!at || (uint32_t)atoi(at + 1) == gn)) {
                         chosen = t;
                         tile_forced = true;
                     }
@@ -1570,6 +1670,10 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     }
     plan_prepends(ks, specs, n, internal, n_internal);
     plan_folds(ks, specs, n, sets, n_sets, internal, n_internal);
+    plan_waves(ks, ctx->compute_units);
+    split_users.erase(std::remove_if(split_users.begin(), split_users.end(),
+                                     [&](const std::pair<size_t, size_t> &u) { return ks->kernels[u.first].per_set[u.second].gemm.ksplit <= 1; }),
+                      split_users.end());
     // The backend's own device memory, one allocation beside the plan's
     // arenas, laid out by lifetime (place_workspace): the packed weights and
     // the attention scratch for the whole program, each split-k GEMM's
@@ -1595,12 +1699,14 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
             for (Launch &L : k.per_set) {
                 if (L.pack < 0) continue;
                 const GemmArgs &g = L.gemm;
-                L.gemm.breg = breg_mode != 0 && L.family == Family::GEMM && (L.math == Math::SPLIT || L.math == Math::F16) &&
+                const bool wave = gemm_tile_wave(L.tile);
+                L.gemm.breg = !wave && breg_mode != 0 && L.family == Family::GEMM && (L.math == Math::SPLIT || L.math == Math::F16) &&
                               g.pipeline && g.load == 0 && g.kgroups == 1 && g.kslices == 2 && g.ksplit <= 1 &&
                               g.k % 64 == 0 && g.k >= 64 && g.k_pad == g.k && (L.tile == TILE_32x64 || L.tile == TILE_64x64) &&
                               (breg_mode == 1 || (g.k >= 2 * g.n && g.k / 64 >= 12));
                 int &v = all[L.pack];
-                v = v < 0 ? (int)L.gemm.breg : (v && L.gemm.breg);
+                const bool frag = wave || L.gemm.breg;
+                v = v < 0 ? (int)frag : (v && frag);
             }
         for (size_t q = 0; q < ks->packs.size(); q++) ks->packs[q].frag = all[q] == 1;
         for (Kernel &k : ks->kernels) {

@@ -283,8 +283,11 @@ hipError_t launch_gemm_f16(const GemmArgs &a, int tile, hipStream_t s);
 hipError_t launch_pack_f32(const PackArgs &a, hipStream_t s);
 hipError_t launch_pack_split(const PackArgs &a, hipStream_t s);
 hipError_t launch_pack_f16(const PackArgs &a, hipStream_t s);
+hipError_t launch_gemm_wave(const GemmArgs &a, Math m, int tile, hipStream_t s);
+inline bool gemm_tile_wave(int t);
 inline hipError_t launch_gemm(const GemmArgs &a, Math m, int tile, hipStream_t s) {
     if (a.row1 <= a.row0) return hipSuccess;
+    if (gemm_tile_wave(tile)) return launch_gemm_wave(a, m, tile, s);
     return m == Math::F32 ? launch_gemm_f32(a, tile, s)
          : m == Math::SPLIT ? launch_gemm_split(a, tile, s) : launch_gemm_f16(a, tile, s);
 }
@@ -343,13 +346,31 @@ __host__ inline uint32_t conv_direct_lds(Math m, uint32_t chunks_held) {
     return planes * (CD_HALO + (chunks_held ? chunks_held : 1) * CD_WTS);
 }
 
+// Whether the wave-split kernel (k_wave.hip) takes this product, its B packed
+// fragment-major: whole 8-column chunks out, no split k, not a fold's consumer
+// and not a projection writing flash operands; A as plain rows of whole
+// 64-wide steps (stored in 16-byte chunks), patches of an image, or a 3x3
+// convolution's windows with at least a k-step of channels in whole 16-byte
+// chunks (split planes only where a k-step stays inside one tap). A staged
+// row's byte offsets are 32-bit.
+__host__ inline bool gemm_wave_fits(const GemmArgs &a, Math m) {
+    const uint32_t epc = m == Math::F16 ? 8 : 4;
+    if (a.n % 8 != 0 || a.ksplit > 1 || a.ln_stats || a.flash_ops || a.row0 >= a.row1) return false;
+    if (a.load == 0) return a.k % 64 == 0 && a.k_pad == a.k && (uint64_t)a.m * a.k * 4 < (1ull << 31);
+    if (a.load == 2) return a.k >= 32;
+    if (a.load != 3 || a.p2 < 32 || a.p2 % epc != 0) return false;
+    return !a.a_planes || (a.p2 % 32 == 0 && (uint64_t)(a.p0 + 1) * (a.p1 + 1) * a.p2 < (1ull << 31) && 9ull * a.p2 < (1u << 16));
+}
+
 // GEMM tile shapes the dispatcher can pick from: BM x BN.
+// TILE_W*: the wave-split kernel's tiles.
 // TILE_CONV3: the direct 3x3 convolution (2 output rows x 64 columns x 32
 // channels per workgroup; its rows and columns below are the pixels and
 // channels of one tile).
-enum GemmTile : int { TILE_64x64 = 0, TILE_32x64 = 1, TILE_64x128 = 2, TILE_128x64 = 3, TILE_128x32 = 4, TILE_64x96 = 5, TILE_CONV3 = 6, TILE_COUNT = 7 };
-inline int gemm_tile_rows(int t) { const int r[] = {64, 32, 64, 128, 128, 64, 128}; return r[t]; }
-inline int gemm_tile_cols(int t) { const int c[] = {64, 64, 128, 64, 32, 96, 32}; return c[t]; }
+enum GemmTile : int { TILE_64x64 = 0, TILE_32x64 = 1, TILE_64x128 = 2, TILE_128x64 = 3, TILE_128x32 = 4, TILE_64x96 = 5, TILE_CONV3 = 6, TILE_W16x32 = 7, TILE_W32x32 = 8, TILE_W32x64 = 9, TILE_COUNT = 10 };
+inline int gemm_tile_rows(int t) { const int r[] = {64, 32, 64, 128, 128, 64, 128, 16, 32, 32}; return r[t]; }
+inline int gemm_tile_cols(int t) { const int c[] = {64, 64, 128, 64, 32, 96, 32, 32, 32, 64}; return c[t]; }
+inline bool gemm_tile_wave(int t) { return t == TILE_W16x32 || t == TILE_W32x32 || t == TILE_W32x64; }
 // K and N of a packed B are padded to these.
 constexpr uint32_t PACK_K = 32, PACK_N = 128;
 
