@@ -422,6 +422,11 @@ struct Fold {
     std::vector<LnStatsArgs> stats;
 };
 
+std::string flash_small_name(Math m, uint32_t blocks) {
+    return std::string(m == Math::F32 ? "mfma-f32" : m == Math::F16 ? "mfma-f16" : "mfma-bf16x3") + " 16x16 queries=" +
+           std::to_string(16 * blocks) + " keys over waves";
+}
+
 const char *main_name(uint32_t m) {
     switch (m) {
     case BL_MAIN_LAYER_NORM: return "layernorm";
@@ -1650,11 +1655,17 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                 L.fl.wgs = fp.wgs;
                 L.fl.units = fp.units;
                 L.fl.merge = fp.merge;
+                // In f16 and bf16x3 the small kernel is for the operands a QKV
+                // projection wrote (below); a flash kernel alone keeps the
+                // 256-query tiles, whose results equal the allocation-free
+                // entry point's bit for bit.
+                L.fl.small = fmath == Math::F32 || getenv("BL_FLASH_SMALL") ? fp.small : 0;
                 L.fl.merge_inline = fp.merge && fp.counters && !getenv("BL_FLASH_MERGE_LAUNCH");
                 scratch_bytes = std::max(scratch_bytes, fp.scratch_bytes);
                 flash_counter_bytes = std::max(flash_counter_bytes, fp.counter_bytes);
                 flash_users.push_back({ki, si});
-                variant = fmath == Math::F32 ? "mfma-f32 splits=" + std::to_string(fp.splits)
+                variant = L.fl.small ? flash_small_name(fmath, fp.small)
+                        : fmath == Math::F32 ? "mfma-f32 splits=" + std::to_string(fp.splits)
                                              : std::string(fmath == Math::F16 ? "mfma-f16" : "mfma-bf16x3") + " 32x32 runs=" +
                                                    std::to_string(fp.wgs) +
                                                    (L.fl.merge_inline ? " merged in-kernel" : fp.merge ? " merged" : "");
@@ -1837,6 +1848,13 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                     ga.fl_tpad = F.fl.t_pad;
                 }
                 F.fl.prepped = 1;
+                if (const uint32_t small = plan_flash(F.math, F.fl.tokens, F.fl.heads, F.fl.row0, F.fl.row1, ctx->compute_units).small) {
+                    F.fl.small = small;
+                    if (si == 0) {
+                        std::string &label = ks->kernels[ki].label;
+                        label.replace(label.find(" @ ") + 3, std::string::npos, flash_small_name(F.math, small));
+                    }
+                }
                 F.kv_producers.assign(producers.begin(), producers.end());
                 std::sort(F.kv_producers.begin(), F.kv_producers.end());
             }

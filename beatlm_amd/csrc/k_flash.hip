@@ -978,6 +978,298 @@ __global__ __launch_bounds__(256) void flash16_merge_kernel(FlashArgs args) {
     }
 }
 
+// ---- 4. few tokens: one workgroup per (head, 16 or 32 queries) ----
+//
+// What bounds attention over a few hundred tokens is latency: the 32 x 32
+// kernel's 256-query tiles leave a handful of tiles, so its runs are one or two
+// key tiles long and their results cross the device's L2s to be merged (12.5 us
+// at 170 to 362 tokens x 6 heads, whatever the tokens; on the f32 matrix cores
+// a prep launch, the kernel and a merge launch). Here the 8 waves of a
+// workgroup split the keys of one head, 32 at a time (wave w: groups w, w + 8,
+// ...), for QB blocks of 16 queries; every wave loads its groups' operands
+// straight into registers, the next group's while one is multiplied, and the 8
+// waves' (max, sum, unnormalised output) meet in LDS. Scores are S^T = K Q^T
+// in 16 x 16 products with the key rows so ordered (small_key) that a lane's
+// 8 scores of query l16 are, as they stand, its B operand of O^T = V^T P^T
+// against 16 consecutive bytes of a Vt row. On the f32 matrix cores K and V come from qkv itself (no prep).
+constexpr int SW = 8, SMALL_THREADS = 64 * SW;
+constexpr int SKEYS = 32;  // keys per group
+constexpr int SROW = HD + 4;
+
+template <Math M> struct SmallKv;
+template <> struct SmallKv<Math::SPLIT> {
+    bf16x8 k[2][2][2];  // [key block][32-wide half of d][plane]
+    bf16x8 v[4][2];     // [16-wide block of d][plane]
+};
+template <> struct SmallKv<Math::F16> {
+    f16x8 k[2][2][1];
+    f16x8 v[4][1];
+};
+template <> struct SmallKv<Math::F32> {
+    f32x4 k[2][4];      // d = 16g + 4i + e
+    float v[2][4][4];   // [key block][key 4g + r][16-wide block of d]
+};
+
+// The key of the group that row i of key block kb holds: a lane's 8 score
+// accumulators (rows 4 g + r of both blocks) are then the keys of positions
+// 8 g .. 8 g + 7 of a Vt row, one 16-byte load.
+__device__ __forceinline__ uint32_t small_key(int i, int kb) { return vt_pos(8 * (i >> 2) + 4 * kb + (i & 3)); }
+
+template <Math M> struct SmallOp;
+template <> struct SmallOp<Math::SPLIT> {
+    using V8 = bf16x8;
+    static __device__ __forceinline__ f32x4 mma(V8 a, V8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+};
+template <> struct SmallOp<Math::F16> {
+    using V8 = f16x8;
+    static __device__ __forceinline__ f32x4 mma(V8 a, V8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+};
+
+template <Math M, int QB>
+__global__ __launch_bounds__(SMALL_THREADS) void attn_small_kernel(FlashArgs a) {
+    using T = typename FlashTraits<M>::T;
+    using L = typename FlashTraits<M>::L;
+    constexpr int PL = M == Math::SPLIT ? 2 : 1;
+    constexpr int QROWS = 16 * QB;
+    __shared__ __attribute__((aligned(16))) float so[SW][QROWS * SROW];
+    __shared__ f32x2 sml[SW][QROWS];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    const uint32_t H = a.heads, Tn = a.tokens, tpad = a.t_pad;
+    // Each XCD takes a contiguous eighth of the (head, query block) order, so
+    // its L2 fetches the keys and values of a head or two.
+    const uint32_t qblocks = (a.row1 - a.row0 + QROWS - 1) / QROWS, total = H * qblocks, per = (total + 7) / 8;
+    const uint32_t idx = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per || idx >= total) return;
+    const uint32_t head = idx / qblocks, q0 = a.row0 + (idx % qblocks) * QROWS;
+    const uint32_t row_stride = 3 * H * HD;
+    const T *qkv = (const T *)a.qkv;
+    const float c = a.scale * LOG2E;
+
+    // The lane's queries (rows past the part re-read its last; never stored).
+    T qraw[QB][16];
+#pragma unroll
+    for (int b = 0; b < QB; b++) {
+        const uint32_t q = min(q0 + 16 * b + l16, a.row1 - 1);
+        const T *qrow = qkv + (uint64_t)q * row_stride + head * HD;
+        // d = 16 g + i on the f32 matrix cores, else 32 (i / 8) + 8 g + i % 8.
+        using Q4 = typename std::conditional<M == Math::F16, f16x4, f32x4>::type;
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+            const Q4 v = *(const Q4 *)(qrow + (M == Math::F32 ? 16 * g + i : 32 * (i / 8) + 8 * g + i % 8));
+#pragma unroll
+            for (int e = 0; e < 4; e++) qraw[b][i + e] = v[e];
+        }
+    }
+
+    const uint64_t plane = (uint64_t)H * tpad * HD;
+    auto load = [&](uint32_t grp, SmallKv<M> &kv) {
+        const uint32_t key0 = SKEYS * grp;
+        if constexpr (M == Math::F32) {
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) {
+                // Keys past the last re-read it: their probabilities are zero.
+                const uint32_t key = min(key0 + 16 * kb + l16, Tn - 1);
+                const float *kp = (const float *)qkv + (uint64_t)key * row_stride + (H + head) * HD + 16 * g;
+#pragma unroll
+                for (int i = 0; i < 4; i++) kv.k[kb][i] = *(const f32x4 *)(kp + 4 * i);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t vkey = min(key0 + 16 * kb + 4 * g + r, Tn - 1);
+                    const float *vp = (const float *)qkv + (uint64_t)vkey * row_stride + (2 * H + head) * HD + l16;
+#pragma unroll
+                    for (int db = 0; db < 4; db++) kv.v[kb][r][db] = vp[16 * db];
+                }
+            }
+        } else {
+            using K8 = typename SmallOp<M>::V8;
+#pragma unroll
+            for (int p = 0; p < PL; p++) {
+#pragma unroll
+                for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                    for (int ds = 0; ds < 2; ds++)
+                        kv.k[kb][ds][p] = *(const K8 *)((const L *)a.kp + p * plane +
+                                                        ((uint64_t)head * tpad + key0 + small_key(l16, kb)) * HD + 32 * ds + 8 * g);
+#pragma unroll
+                for (int db = 0; db < 4; db++)
+                    kv.v[db][p] = *(const K8 *)((const L *)a.vt + p * plane + ((uint64_t)head * HD + 16 * db + l16) * tpad + key0 + 8 * g);
+            }
+        }
+    };
+
+    f32x4 o[QB][4];  // O^T: d = 16 db + 4g + r, query 16 b + l16
+    float m[QB], l[QB];
+#pragma unroll
+    for (int b = 0; b < QB; b++) {
+        m[b] = -INFINITY;
+        l[b] = 0.0f;
+#pragma unroll
+        for (int db = 0; db < 4; db++) o[b][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    // The queries as operands, scaled by scale * log2(e) first but on the f32
+    // matrix cores (whose scores are scaled).
+    using Q8 = typename std::conditional<M == Math::SPLIT, bf16x8, f16x8>::type;
+    Q8 qh[QB][2], ql[QB][2];
+    auto prepare_q = [&]() {
+        if constexpr (M != Math::F32) {
+#pragma unroll
+            for (int b = 0; b < QB; b++)
+#pragma unroll
+                for (int ds = 0; ds < 2; ds++) {
+                    float qv[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) qv[e] = to_f32(qraw[b][8 * ds + e]) * c;
+                    if constexpr (M == Math::SPLIT) {
+                        split8_bf16(qv, qh[b][ds], ql[b][ds]);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) qh[b][ds][e] = (_Float16)qv[e];
+                    }
+                }
+        }
+    };
+
+    auto step = [&](uint32_t grp, const SmallKv<M> &kv) {
+        const uint32_t key0 = SKEYS * grp;
+#pragma unroll
+        for (int b = 0; b < QB; b++) {
+            f32x4 s[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++) {
+                if constexpr (M == Math::F32) {
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.k[kb][i / 4][i % 4], qraw[b][i], s[kb], 0, 0, 0);
+                    s[kb] *= c;
+                } else {
+#pragma unroll
+                    for (int ds = 0; ds < 2; ds++) {
+                        if constexpr (M == Math::SPLIT) {
+                            s[kb] = SmallOp<M>::mma(kv.k[kb][ds][1], qh[b][ds], s[kb]);
+                            s[kb] = SmallOp<M>::mma(kv.k[kb][ds][0], ql[b][ds], s[kb]);
+                        }
+                        s[kb] = SmallOp<M>::mma(kv.k[kb][ds][0], qh[b][ds], s[kb]);
+                    }
+                }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    if (key0 + (M == Math::F32 ? 16 * kb + 4 * g + r : small_key(4 * g + r, kb)) >= Tn) s[kb][r] = -INFINITY;
+                    mx = fmaxf(mx, s[kb][r]);
+                }
+            mx = max_xor32(fmaxf(mx, __shfl_xor(mx, 16, WAVE)));
+            const float m_new = fmaxf(m[b], mx);  // finite: every group holds a key < T
+            const float alpha = __builtin_amdgcn_exp2f(m[b] - m_new);
+            m[b] = m_new;
+            float p[8], sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                p[e] = __builtin_amdgcn_exp2f(s[e / 4][e % 4] - m_new);
+                if constexpr (M == Math::F16) p[e] = (float)(_Float16)p[e];
+                sum += p[e];
+            }
+            l[b] = l[b] * alpha + sum;
+#pragma unroll
+            for (int db = 0; db < 4; db++) o[b][db] *= alpha;
+            if constexpr (M == Math::F32) {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int db = 0; db < 4; db++)
+                        o[b][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.v[e / 4][e % 4][db], p[e], o[b][db], 0, 0, 0);
+            } else {
+                using V8 = typename SmallOp<M>::V8;
+                V8 ph, pl;
+                if constexpr (M == Math::SPLIT) {
+                    split8_bf16(p, ph, pl);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) ph[e] = (_Float16)p[e];
+                }
+#pragma unroll
+                for (int db = 0; db < 4; db++) {
+                    if constexpr (M == Math::SPLIT) {
+                        o[b][db] = SmallOp<M>::mma(kv.v[db][1], ph, o[b][db]);
+                        o[b][db] = SmallOp<M>::mma(kv.v[db][0], pl, o[b][db]);
+                    }
+                    o[b][db] = SmallOp<M>::mma(kv.v[db][0], ph, o[b][db]);
+                }
+            }
+        }
+    };
+
+    const uint32_t groups = (Tn + SKEYS - 1) / SKEYS;
+    SmallKv<M> kva, kvb;
+    uint32_t j = wave;
+    if (j < groups) load(j, kva);
+    prepare_q();
+    for (; j < groups; j += 2 * SW) {
+        if (j + SW < groups) load(j + SW, kvb);
+        step(j, kva);
+        if (j + SW < groups) {
+            if (j + 2 * SW < groups) load(j + 2 * SW, kva);
+            step(j + SW, kvb);
+        }
+    }
+
+#pragma unroll
+    for (int b = 0; b < QB; b++) {
+        const float lt = sum_xor32(l[b] + __shfl_xor(l[b], 16, WAVE));
+        if (g == 0) sml[wave][16 * b + l16] = f32x2{m[b], lt};
+#pragma unroll
+        for (int db = 0; db < 4; db++) *(f32x4 *)&so[wave][(16 * b + l16) * SROW + 16 * db + 4 * g] = o[b][db];
+    }
+    __syncthreads();
+    // Four columns of one query an invocation, the waves in order.
+    if (tid >= QROWS * (HD / 4)) return;
+    const uint32_t r = tid / (HD / 4), d = tid % (HD / 4) * 4, q = q0 + r;
+    float mt = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < SW; w++) mt = fmaxf(mt, sml[w][r][0]);
+    float lt = 0.0f;
+    f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < SW; w++) {
+        const f32x2 ml = sml[w][r];
+        const float wt = __builtin_amdgcn_exp2f(ml[0] - mt);  // 0 for a wave without keys
+        lt += ml[1] * wt;
+        acc += *(const f32x4 *)&so[w][r * SROW + d] * wt;
+    }
+    if (q >= a.row1) return;
+    const float inv = 1.0f / lt;
+    if constexpr (M == Math::F16) {
+        f16x4 w4;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w4[e] = (_Float16)(acc[e] * inv);
+        *(f16x4 *)((T *)a.out + ((uint64_t)q * H + head) * HD + d) = w4;
+    } else {
+        store_f32x4((float *)a.out, ((uint64_t)q * H + head) * HD + d, acc * inv, a.out_planes);
+    }
+}
+
+template <Math M>
+hipError_t launch_small(const FlashArgs &a, hipStream_t s) {
+    if constexpr (M != Math::F32) {
+        if (!a.prepped) {
+            hipLaunchKernelGGL((flash_prep_kernel<M, true>), dim3(a.t_pad / KT, a.heads), dim3(THREADS), 0, s, a);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+    }
+    const uint32_t rows = a.row1 - a.row0, qrows = 16 * a.small, total = (rows + qrows - 1) / qrows * a.heads;
+    const dim3 grid((total + 7) / 8 * 8), block(SMALL_THREADS);
+    if (a.small == 1) hipLaunchKernelGGL((attn_small_kernel<M, 1>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((attn_small_kernel<M, 2>), grid, block, 0, s, a);
+    return hipGetLastError();
+}
+
 constexpr uint32_t FLASH16_MAX_SPLITS = 8;
 
 uint64_t operand_bytes(Math m, uint32_t heads, uint32_t t_pad) {
@@ -1019,11 +1311,31 @@ hipError_t launch_16(const FlashArgs &a, hipStream_t s) {
 
 hipError_t launch_flash(const FlashArgs &a, Math m, hipStream_t s) {
     if (a.row1 <= a.row0) return hipSuccess;
+    if (a.small)
+        return m == Math::F16 ? launch_small<Math::F16>(a, s) : m == Math::SPLIT ? launch_small<Math::SPLIT>(a, s) : launch_small<Math::F32>(a, s);
     switch (m) {
     case Math::F16: return launch_32<Math::F16>(a, s);
     case Math::SPLIT: return launch_32<Math::SPLIT>(a, s);
     default: return launch_16(a, s);
     }
+}
+
+// 16-query blocks per workgroup of attn_small_kernel, 0 for the other kernels:
+// the fewest (1 or 2) whose workgroups all run at once, one per CU; a second
+// round doubles its time. It beats the 256-query tiles over all such sizes in
+// f16 (us, 256-query tiles / 1 block / 2 blocks; 6 heads: 257 tokens 11.4 /
+// 5.0 / 6.0, 626 12.9 / 7.2 / 8.4, 1200 16.0 / 21.2 / 13.2; 16 heads, 500: 15.2
+// / 10.8 / 7.2) and on the f32 matrix cores (257: 17.2 / 9.3 / 14.3; 1025: 38.7
+// / 37.8 / 30.4); in bf16x3, whose keys and values are twice the bytes, up to
+// 640 tokens (6 heads: 257 12.6 / 7.7 / 9.4, 626 14.2 / 12.3 / 14.0, 700 15.1 /
+// 25.7 / 15.5; 12 heads, 626: 15.7 / 23.4 / 14.3). BL_FLASH_SMALL: 0, 1 or 2
+// blocks whatever the size.
+static uint32_t small_blocks(Math m, uint32_t tokens, uint32_t heads, uint32_t rows, uint32_t compute_units) {
+    if (const char *knob = getenv("BL_FLASH_SMALL")) return std::min(2, std::max(0, atoi(knob)));
+    if (getenv("BL_FLASH_MERGE_LAUNCH") || (m == Math::SPLIT && tokens > 640)) return 0;
+    for (uint32_t b = 1; b <= 2; b++)
+        if ((uint64_t)heads * ((rows + 16 * b - 1) / (16 * b)) <= compute_units) return b;
+    return 0;
 }
 
 FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uint32_t row1, uint32_t compute_units) {
@@ -1032,6 +1344,7 @@ FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uin
     const uint32_t t_pad = (tokens + KT - 1) / KT * KT;
     const uint32_t kt = t_pad / KT;
     uint64_t extra = 0;
+    p.small = small_blocks(m, tokens, heads, rows, compute_units);
     if (m == Math::F32) {
         const uint32_t wgs = (rows + 63) / 64 * heads;
         // Enough workgroups for two per CU, each split keeping two key tiles or more.

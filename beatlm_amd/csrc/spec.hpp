@@ -205,12 +205,15 @@ struct FlashArgs {
     // per (head, query tile) pair; every counter is zero between launches.
     uint32_t merge_inline;
     uint32_t *counters;
+    // Few tokens: 16-query blocks per workgroup of the kernel whose waves
+    // split the keys (1 or 2; it needs no partial results); 0: the others.
+    uint32_t small;
 };
 
 // How a flash attention spec is launched: its grid and the scratch it needs
 // (operands, then partial outputs and statistics).
 struct FlashPlan {
-    uint32_t splits = 1, qtiles = 0, wgs = 0, merge = 0;
+    uint32_t splits = 1, qtiles = 0, wgs = 0, merge = 0, small = 0;
     uint64_t units = 0;
     // Operands, partial results and statistics. The arrival counters of the
     // in-kernel merge (`counters` words, one per (head, query tile) pair) are

@@ -122,6 +122,7 @@ extern "C" int bl_flash_attention_static(bl_ctx *ctx, const void *qkv, void *out
     a.wgs = plan.wgs;
     a.units = plan.units;
     a.merge = plan.merge;
+    a.small = m == bl::Math::F32 ? plan.small : 0;  // as bl_kernels_encode without a projection before it
     a.merge_inline = plan.merge && plan.counters;
     a.prepped = 0;  // the prep launch writes K and Vt into the scratch
     bl::bind_flash_scratch(a, m, base, COUNTER_BYTES);

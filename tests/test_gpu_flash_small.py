@@ -1,0 +1,92 @@
+"""The flash attention kernel for few tokens (one workgroup per head and 16 or
+32 queries, its waves splitting the keys in groups of 32) against the oracle:
+one token, tokens that end inside a query block, a key group and a round of
+eight groups, exactly on them, and three rounds; a kernel of several parts;
+and a block whose attention reads the operands its QKV projection wrote.
+
+Tolerance for f32 storage: |got - want| <= 1e-4 + 1e-4 |want|
+(reference.rs:22-24); for f16 storage, max abs error <= 2e-2 against the
+oracle on the same f16-rounded inputs.
+"""
+
+import numpy as np
+import pytest
+
+import oracle
+from beatlm_amd import hip, ir
+from tests.blockdata import block_graph, block_values, block_weights, max_abs_err
+from tests.test_gpu_sweep import attention_graph
+
+pytestmark = pytest.mark.gpu
+
+X, Y = 0, 20
+F16_TOL = 2e-2
+MATHS = ["bf16x3", "f32", "f16"]
+
+
+def compare(got, want, math, what):
+    if math == "f16":
+        err = max_abs_err(got, want)
+        assert err <= F16_TOL, f"{what}: max abs error {err:.3e}"
+    else:
+        bad = oracle.first_mismatch(got, want)
+        assert bad is None, f"{what}: element {bad[0]} is {bad[1]}, the oracle says {bad[2]}"
+
+
+@pytest.fixture
+def math(ctx, request):
+    if request.param == "f32":
+        ctx.set_f32_math(hip.F32_MATH_MFMA_F32)
+    yield request.param
+    ctx.set_f32_math(hip.F32_MATH_SPLIT_BF16)
+
+
+@pytest.mark.parametrize("t,h,parts", [(1, 1, 1), (15, 2, 1), (32, 1, 1), (33, 3, 1), (64, 2, 1), (256, 1, 1), (257, 6, 1),
+                                       (290, 2, 3), (700, 2, 1)])
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+@pytest.mark.parametrize("blocks", ["1", "2"])
+def test_attention_of_few_tokens_matches_the_oracle(ctx, monkeypatch, t, h, parts, math, blocks):
+    monkeypatch.setenv("BL_FLASH_SMALL", blocks)
+    # Scores of up to +-40, so that the running maximum moves and most
+    # probabilities are small.
+    qkv = oracle.uniform(t + 100 * h, t * 3 * h * 64, -3.0, 3.0)
+    if math == "f16":
+        qkv = qkv.astype(np.float16)
+    want = oracle.attention(qkv.astype(np.float32), t, h, 64, 0.125)
+    prep = ir.prepare(ctx, attention_graph(t, h, 64), parts=parts, dtype=hip.F16 if math == "f16" else hip.F32)
+    try:
+        assert all("keys over waves" in prep.kernels.label(k) for k in range(len(prep.kernels)))
+        prep.write(X, qkv)
+        prep.run()
+        ctx.synchronize()
+        compare(prep.read(Y).astype(np.float32), want, math, f"t={t} h={h} parts={parts}")
+    finally:
+        prep.close()
+
+
+@pytest.mark.parametrize("t", [50, 257])
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+def test_a_small_blocks_attention_reads_its_projections_operands(ctx, t, math):
+    """The planner's own choice in an encoder block, run twice (the second pass
+    finds the first one's operands and statistics)."""
+    d, h, mlp = 128, 2, 512
+    x, w = oracle.uniform(21, t * d, -2.0, 2.0), block_weights(d, mlp, 100, "reference")
+    g, ids = block_graph(t, d, h, mlp, 1e-6)
+    prep = ir.prepare(ctx, g, dtype=hip.F16 if math == "f16" else hip.F32)
+    try:
+        labels = [prep.kernels.label(k) for k in range(len(prep.kernels))]
+        assert any("keys over waves" in lab for lab in labels), labels
+        vals = block_values(ids, x, w)
+        if math == "f16":
+            vals = {k: v.astype(np.float16) for k, v in vals.items()}
+        for tid, v in vals.items():
+            prep.write(tid, v)
+        for _ in range(2):
+            prep.run()
+        ctx.synchronize()
+        got = prep.read(ids.output).astype(np.float32)
+    finally:
+        prep.close()
+    if math == "f16":
+        x, w = (x.astype(np.float16).astype(np.float32), {k: v.astype(np.float16).astype(np.float32) for k, v in w.items()})
+    compare(got, oracle.vit_block(x, w, t, h, d // h, mlp, 1e-6), math, f"block of {t} tokens")
