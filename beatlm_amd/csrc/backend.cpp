@@ -1481,10 +1481,14 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                     else chosen = (gn >= 1024 && w64 <= 2ull * ctx->compute_units) ? TILE_64x64 : TILE_32x64;
                     // bf16x3 outputs of whole 96-column tiles, at least 1536
                     // wide, that fit one round at two 64 x 96 workgroups per CU
-                    // (fc1 at the encoder's sizes: 13.3 -> 12.3 us against 32 x
-                    // 64 in two rounds; QKV's 1152 columns measured slower
-                    // than its 64 x 64 tiles, 11.3 -> 12.1).
-                    if (fmath == Math::SPLIT && gn >= 1536 && gn % 96 == 0 &&
+                    // where 64 x 64 ones do not (fc1 384 -> 1536 at 1370
+                    // tokens: 13.3 -> 12.3 us against 32 x 64 in two rounds;
+                    // QKV's 1152 columns measured slower than its 64 x 64
+                    // tiles, 11.3 -> 12.1). Where 64 x 64 tiles fit a round
+                    // too they leave fewer CUs idle (64 x 96 / 64 x 64: fc1 at
+                    // 362 tokens 10.8 / 8.2, 626 11.5 / 8.6, 1025 13.7 / 11.5;
+                    // 768 -> 3072 at 626 22.5 / 19.1).
+                    if (fmath == Math::SPLIT && gn >= 1536 && gn % 96 == 0 && w64 > 2ull * ctx->compute_units &&
                         wgs_of(TILE_64x96) <= 2ull * ctx->compute_units && !getenv("BL_GEMM_NO_96"))
                         chosen = TILE_64x96;
                 }
