@@ -985,14 +985,21 @@ void plan_folds(bl_kernels *ks, const bl_spec *specs, uint32_t n, const bl_bindi
 //                            over 74 x 74: 15.2 / 12.0 / 14.3 / 9.5
 //   patch embedding 588 -> 384, 169 patches: 16.9 / 5.8 / 7.6 / 10.7
 // Weights beyond an XCD's L2 (6 MB: 4096 -> 1024) come from further away for
-// every row of tiles: 32 rows at least (f16, 65 tokens: 17.9 / 9.2 / 7.1). A
-// product of one 64-wide step takes the 32 x 64 ring tile rather than the
-// same tile here (74 x 74 x 64 -> 64: 4.1 against 4.5). The f32 matrix cores
-// are slow enough that long products want more workgroups than one per
-// tile: convolutions of more than 2048 keep split k (384 -> 64 over 13 x 13:
-// 12.3 against 15.1), and the 32 x 64 tile is only for products longer than
-// 512 (QKV at 257 tokens: 8.2 against 8.5). BL_GEMM_WAVE: 0 none, 1 .. 3 that
-// tile wherever the kernel takes the product.
+// every row of tiles: 32 rows at least (f16, 65 tokens: 17.9 / 9.2 / 7.1), and
+// a wide product of such weights reads them better in the ring (fc1 1024 ->
+// 4096 in bf16x3, 65 tokens: 11.9 against 13.6). In f16 a k of one step a wave
+// leaves LDS and registers for two 32 x 32 workgroups per CU, so twice the
+// tiles run at once (QKV 384 -> 1152, 443 tokens, 504 tiles: 5.8 against 4.1;
+// bf16x3 at 257 tokens, 324 tiles: 6.7 against 7.3, and 5.9 with 32 x 64). A
+// product of one 64-wide step takes the 32 x 64 ring tile rather than the same
+// tile here (74 x 74 x 64 -> 64: 4.1 against 4.5). The f32 matrix cores are
+// slow enough that long products want more workgroups than one per tile:
+// convolutions of more than 2048 keep split k (384 -> 64 over 13 x 13: 12.3
+// against 15.1), and the 32 x 64 tile is only for products longer than 512
+// (QKV at 257 tokens: 8.2 against 8.5). Folded LayerNorms' consumers gain less,
+// their rings being short: QKV at 170 tokens 6.7 -> 4.8, at 257 6.7 -> 5.9,
+// fc1 at 257 7.2 -> 7.0. BL_GEMM_WAVE: 0 none, 1 .. 3 that tile wherever the
+// kernel takes the product.
 int wave_tile_of(const GemmArgs &g, Math m, uint32_t compute_units, int mode) {
     const int tiles[] = {TILE_W16x32, TILE_W32x32, TILE_W32x64};
     if (mode >= 1 && mode <= 3) return tiles[mode - 1];
@@ -1000,17 +1007,17 @@ int wave_tile_of(const GemmArgs &g, Math m, uint32_t compute_units, int mode) {
     if (m == Math::F32 && g.load == 3 && g.k > 2048) return -1;
     for (int t : tiles) {
         if (t == TILE_W16x32 && weight_bytes > (6u << 20) && g.row1 - g.row0 > 16) continue;
-        if (t == TILE_W32x64 && (g.k <= 64 || (m == Math::F32 && g.k <= 512))) continue;
+        if (t == TILE_W32x64 && (g.k <= 64 || (m == Math::F32 && g.k <= 512) || (weight_bytes > (12u << 20) && g.n > g.k))) continue;
+        const uint64_t at_once = m == Math::F16 && g.load == 0 && t == TILE_W32x32 && g.k <= 512 ? 2ull * compute_units : compute_units;
         const uint64_t rows = (g.row1 - g.row0 + gemm_tile_rows(t) - 1) / gemm_tile_rows(t);
-        if (rows * ((g.n + gemm_tile_cols(t) - 1) / gemm_tile_cols(t)) <= compute_units) return t;
+        if (rows * ((g.n + gemm_tile_cols(t) - 1) / gemm_tile_cols(t)) <= at_once) return t;
     }
     return -1;
 }
 
 // Gives products to the wave-split kernel (k_wave.hip) where wave_tile_of says
 // so, in every binding set, in place of a ring or of a split k and its reduce
-// launch. Not a projection that writes a flash kernel's operands, nor the
-// consumer of a folded LayerNorm.
+// launch.
 void plan_waves(bl_kernels *ks, uint32_t compute_units) {
     const char *knob = getenv("BL_GEMM_WAVE");
     const int mode = knob ? atoi(knob) : -1;
@@ -1029,11 +1036,8 @@ void plan_waves(bl_kernels *ks, uint32_t compute_units) {
             int t = -1;
             GemmArgs g = L.gemm;
             g.ksplit = 1;
-            if (L.family == Family::GEMM && g.pipeline && L.tile != TILE_CONV3 && L.fold_role != FOLD_CONSUMER && gemm_wave_fits(g, L.math))
+            if (L.family == Family::GEMM && g.pipeline && L.tile != TILE_CONV3 && gemm_wave_fits(g, L.math))
                 t = wave_tile_of(g, L.math, compute_units, mode);
-            // A projection of a flash kernel that takes its operands from it.
-            for (const Kernel &o : ks->kernels)
-                if (o.per_set[si].family == Family::FLASH && o.per_set[si].math != Math::F32 && o.per_set[si].fl.qkv == g.c) t = -1;
             if (si == 0) tile = t;
             else if (t != tile) tile = -1;
         }

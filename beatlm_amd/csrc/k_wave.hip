@@ -110,8 +110,10 @@ __device__ __forceinline__ void wave_take(WaveA<M, TM> &a, int i, const float (&
 // LOAD: 0 plain rows, 2 the patch gather, 3 the 3x3 convolution's windows.
 // AP: A kept as hi and lo bf16 planes (bf16x3). KS: 32-wide slices per k-step.
 // NS: steps of a wave in flight at once.
-template <Math M, int BM, int BN, int LOAD, bool AP, int KS, int NS>
-__global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
+// FOLD: the consumer of a folded LayerNorm (plain rows; it has no bias, and its
+// epilogue's operands are loaded where they are used).
+template <Math M, int BM, int BN, int LOAD, bool AP, int KS, int NS, bool FOLD = false>
+__global__ __launch_bounds__(WV_THREADS, NS == 1 && BN == 32 ? 4 : 2) void gemm_wave_kernel(GemmArgs args) {
     using T = typename GemmTraits<M>::T;
     static_assert(!AP || (M == Math::SPLIT && LOAD != 2), "split A planes feed the bf16x3 math");
     static_assert(LOAD != 2 || KS == 1, "the patch gather takes one slice a step");
@@ -147,12 +149,32 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
     bias.zero();
     op0.zero();
     op1.zero();
+    // A folded LayerNorm's consumer (plain rows): the row's block statistics (a
+    // quad's lane every fourth pair of blocks, as fold_load takes them), d and c.
+    f32x4 stats[FOLD ? FOLD_PER : 1];
+    Raw8<float> fd, fc;
+    if constexpr (FOLD) {
+        fd.zero();
+        fc.zero();
+        if (chunk) {
+            const f32x4 *st = (const f32x4 *)(args.ln_stats + 2 * (uint64_t)min(row, row_end - 1) * args.ln_blocks);
+#pragma unroll
+            for (int q = 0; q < FOLD_PER; q++) {
+                const uint32_t b = cc % 4 + 4 * q;
+                stats[q] = b < args.ln_blocks / 2 ? st[b] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            if (col < N) {
+                fd.load(args.ln_d + col);
+                if (M == Math::F16) fc.load(args.ln_c + col);
+            }
+        }
+    }
     const EpilogueArgs &epi = args.epi;
     auto operand8 = [&](int s, Raw8<T> &r) {
         if (epi.kind[s] == BL_EPI_ADD) r.load((const T *)epi.operand[s] + idx);
         else if (epi.kind[s] == BL_EPI_CHANNEL_SCALE && epi.channels[s] == N) r.load((const T *)epi.operand[s] + col);
     };
-    if (live) {
+    if (!FOLD && live) {
         if (args.bias) bias.load((const T *)args.bias + col);
         if (epi.n > 0) operand8(0, op0);
         if (epi.n > 1) operand8(1, op1);
@@ -238,6 +260,51 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
             else return Loader(K * AESZ, a_limit, 0, lane, AP ? (uint32_t)(args.a_planes * 2) : 0u);
         };
         const Loader load = make();
+        if constexpr (FOLD && M != Math::F16) {
+            // A centred fold's correction (fold_correct) from the last wave,
+            // which has the fewest steps: delta[row][block] = the block's mean
+            // less the row's, times cb, one more 32-deep slice. Lane group g
+            // holds blocks 8 g .. 8 g + 7 of both.
+            if (wave == WV_WAVES - 1) {
+                WaveA<M, TM> da;
+                WaveB<M, TN> cb;
+                const uint32_t nb = args.ln_blocks;
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+                    const uint32_t r = m0 + min((uint32_t)(16 * i + l16), a_limit);
+                    const f32x4 *st = (const f32x4 *)(args.ln_stats + 2 * ((uint64_t)r * nb + 8 * g));
+                    float d[8], sum = 0.0f;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const f32x4 x = 8 * g + 2 * q < nb ? st[q] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                        d[2 * q] = x[0];
+                        d[2 * q + 1] = x[2];
+                        sum += x[0] + x[2];
+                    }
+                    sum += __shfl_xor(sum, 16, WAVE);
+                    sum += __shfl_xor(sum, 32, WAVE);
+                    const float mean = sum / (float)nb;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) d[e] = 8 * g + e < nb ? d[e] - mean : 0.0f;
+                    wave_take<M, TM>(da, i, d);
+                }
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const f32x4 *p = (const f32x4 *)(args.ln_cb + (uint64_t)(n0 + 16 * j + l16) * 32 + 8 * g);
+                    const f32x4 c0 = p[0], c1 = p[1];
+                    if constexpr (M == Math::F32) {
+                        cb.v[0][j] = c0;
+                        cb.v[1][j] = c1;
+                    } else {
+                        float c[8];
+#pragma unroll
+                        for (int e = 0; e < 8; e++) c[e] = e < 4 ? c0[e] : c1[e - 4];
+                        split8_bf16(c, cb.v[0][j], cb.v[1][j]);
+                    }
+                }
+                wave_mma<M, TM, TN>(acc, da, cb);
+            }
+        }
         const char *Ab = (const char *)args.a + (uint64_t)m0 * K * AESZ;
         constexpr int AROWB = A_CPR * 16;
         const int xa = swz<A_CPR>(l16, 0);
@@ -315,7 +382,11 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
             for (int r = 0; r < 4; r++) part[(16 * i + 4 * g + r) * TROW + 16 * j + l16] = acc[i][j][r];
     __syncthreads();
     if (LOAD == 2 && args.cls_out && m0 == args.row0 && wave == WV_WAVES - 1) cls_row<M, T>(args, n0, BN, lane);  // x's first row
-    if (!chunk) return;
+    // The attention's operands: K and V columns of a QKV projection.
+    constexpr bool FLASH = LOAD == 0 && M != Math::F32;
+    const uint32_t D = N / 3;
+    const bool k_region = FLASH && args.flash_ops && n0 >= D && n0 < 2 * D, v_region = FLASH && args.flash_ops && n0 >= 2 * D;
+    if (chunk) {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = 0.0f;
@@ -326,6 +397,22 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
 #pragma unroll
         for (int e = 0; e < 8; e++) v[e] += e < 4 ? x0[e] : x1[e - 4];
     }
+    if constexpr (FOLD) {
+        // The row's mean and variance from its blocks', as fold_finish.
+        float s = 0.0f, m2 = 0.0f;
+#pragma unroll
+        for (int q = 0; q < FOLD_PER; q++) s += stats[q][0] + stats[q][2];
+        const float mean = quad_sum(s) * (1.0f / (float)args.ln_blocks);
+#pragma unroll
+        for (int q = 0; q < FOLD_PER; q++) {
+            const float d0 = stats[q][0] - mean, d1 = stats[q][2] - mean;
+            if (cc % 4 + 4 * q < args.ln_blocks / 2) m2 += stats[q][1] + stats[q][3] + 32.0f * (d0 * d0 + d1 * d1);
+        }
+        m2 = quad_sum(m2);
+        const float rstd = 1.0f / sqrtf(m2 / (float)(32 * args.ln_blocks) + args.ln_eps), shift = M == Math::F16 ? mean : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = rstd * (v[e] - (M == Math::F16 ? shift * fc.at(e) : 0.0f)) + fd.at(e);
+    }
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] += bias.at(e);
     if (live) {
@@ -334,12 +421,12 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
             const int kind = epi.kind[st];
             if (kind == BL_EPI_ADD) {
                 Raw8<T> o = st == 0 ? op0 : op1;
-                if (st > 1) o.load((const T *)epi.operand[st] + idx);
+                if (FOLD || st > 1) o.load((const T *)epi.operand[st] + idx);
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[e] += o.at(e);
             } else if (kind == BL_EPI_CHANNEL_SCALE && epi.channels[st] == N) {
                 Raw8<T> o = st == 0 ? op0 : op1;
-                if (st > 1) o.load((const T *)epi.operand[st] + col);
+                if (FOLD || st > 1) o.load((const T *)epi.operand[st] + col);
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[e] *= o.at(e);
             } else if (kind == BL_EPI_CHANNEL_SCALE) {
@@ -356,7 +443,20 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
             }
         }
     }
-    if (live) store8<T>((T *)args.c, idx, v, args.c_planes);
+    if (live && !(args.flash_ops == 2 && (k_region || v_region))) store8<T>((T *)args.c, idx, v, args.c_planes);
+    if constexpr (FLASH) {
+        if (k_region && live) {
+            const uint32_t kc = col - D;
+            store8_operand<M>(args.fl_kp, ((uint64_t)(kc / 64) * args.fl_tpad + row) * 64 + kc % 64, v,
+                              (uint64_t)(D / 64) * args.fl_tpad * 64);
+        }
+        if (v_region) {
+            // Into wave 0's partial tile (this invocation's own chunk) for the pass by columns.
+            float *t = (float *)smem + tr * TROW + 8 * cc;
+            *(f32x4 *)t = f32x4{v[0], v[1], v[2], v[3]};
+            *(f32x4 *)(t + 4) = f32x4{v[4], v[5], v[6], v[7]};
+        }
+    }
     if (args.ln_out) {
         // A fold's producer: the 32-column block of the values as stored is
         // the 4 chunks of one quad.
@@ -381,21 +481,77 @@ __global__ __launch_bounds__(WV_THREADS) void gemm_wave_kernel(GemmArgs args) {
                 store8<T>((T *)args.ln_shadow, idx, dv, M == Math::SPLIT ? (args.ln_plane ? args.ln_plane : (uint64_t)args.m * N) : 0);
             }
     }
+    }
+    if constexpr (FLASH) {
+        if (v_region) {
+            // Column cl, 16 tokens, as chunk_epilogue writes them: m0 is a
+            // multiple of 16, position s of the run holds token vt_pos(s).
+            __syncthreads();
+            const float *tile = (const float *)smem;
+            const uint64_t plane = (uint64_t)(D / 64) * args.fl_tpad * 64;
+            if (tid < BN * (BM / 16)) {
+                const int cl = tid % BN, tr0 = tid / BN * 16;
+                const uint32_t row0 = m0 + tr0, vc = n0 + cl - 2 * D;
+                const uint64_t base = (uint64_t)vc * args.fl_tpad;
+                if (row0 < row_end) {
+                    float y0[8], y1[8];
+#pragma unroll
+                    for (int s = 0; s < 8; s++) {
+                        y0[s] = tile[(tr0 + vt_pos(s)) * TROW + cl];
+                        y1[s] = tile[(tr0 + vt_pos(s + 8)) * TROW + cl];
+                    }
+                    if (row0 + 16 <= row_end) {
+                        store8_operand<M>(args.fl_vt, base + row0, y0, plane);
+                        store8_operand<M>(args.fl_vt, base + row0 + 8, y1, plane);
+                    } else {
+#pragma unroll
+                        for (int s = 0; s < 16; s++) {
+                            if (row0 + vt_pos(s) >= row_end) continue;
+                            const float x = s < 8 ? y0[s] : y1[s - 8];
+                            const uint64_t i = base + row0 + s;
+                            if constexpr (M == Math::SPLIT) {
+                                __bf16 h, l;
+                                split_bf16(x, h, l);
+                                ((__bf16 *)args.fl_vt)[i] = h;
+                                ((__bf16 *)args.fl_vt)[plane + i] = l;
+                            } else {
+                                ((_Float16 *)args.fl_vt)[i] = (_Float16)x;
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
 }
 
 template <Math M, int BM, int BN, int LOAD, bool AP, int KS>
 hipError_t wave_ns(const GemmArgs &a, hipStream_t s) {
     const dim3 grid(xcd_grid(BM, BN, a)), block(WV_THREADS);
+    if constexpr (LOAD == 0) {
+        // x of at most 1024 columns: one or two steps a wave.
+        if (a.ln_stats) {
+            if (a.k <= 64 * WV_WAVES) hipLaunchKernelGGL((gemm_wave_kernel<M, BM, BN, LOAD, AP, KS, 1, true>), grid, block, 0, s, a);
+            else hipLaunchKernelGGL((gemm_wave_kernel<M, BM, BN, LOAD, AP, KS, 2, true>), grid, block, 0, s, a);
+            return hipGetLastError();
+        }
+    }
     if constexpr (LOAD == 2) {
-        hipLaunchKernelGGL((gemm_wave_kernel<M, BM, BN, LOAD, AP, KS, 4>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((gemm_wave_kernel<M, BM, BN, LOAD, AP, KS, 3>), grid, block, 0, s, a);
     } else {
-        // As many steps a wave in flight as it has, where LDS holds them: 2
-        // (half the LDS, so two workgroups fit a CU), 4, or 8.
+        // As many steps a wave in flight as it has, where LDS holds them: 1 or
+        // 2 (so that two workgroups fit a CU), 4, or 8.
         constexpr int STAGE = WV_WAVES * BM * PipeTraits<M>::A_CPR * KS * 16;
         const uint32_t n = (a.k_pad / (32 * KS) + WV_WAVES - 1) / WV_WAVES;
         if constexpr (M == Math::F16 && 8 * STAGE <= 160 * 1024 && LOAD == 0) {
             if (n > 4) {
                 hipLaunchKernelGGL((gemm_wave_kernel<M, BM, BN, LOAD, AP, KS, 8>), grid, block, 0, s, a);
+                return hipGetLastError();
+            }
+        }
+        if constexpr (M == Math::F16 && BM == 32 && BN == 32 && LOAD == 0) {
+            if (n == 1) {
+                hipLaunchKernelGGL((gemm_wave_kernel<M, BM, BN, LOAD, AP, KS, 1>), grid, block, 0, s, a);
                 return hipGetLastError();
             }
         }

@@ -350,15 +350,17 @@ __host__ inline uint32_t conv_direct_lds(Math m, uint32_t chunks_held) {
 }
 
 // Whether the wave-split kernel (k_wave.hip) takes this product, its B packed
-// fragment-major: whole 8-column chunks out, no split k, not a fold's consumer
-// and not a projection writing flash operands; A as plain rows of whole
-// 64-wide steps (stored in 16-byte chunks), patches of an image, or a 3x3
-// convolution's windows with at least a k-step of channels in whole 16-byte
-// chunks (split planes only where a k-step stays inside one tap). A staged
-// row's byte offsets are 32-bit.
+// fragment-major: whole 8-column chunks out, no split k; A as plain rows of
+// whole 64-wide steps (a folded LayerNorm's consumer and a projection writing
+// flash operands among them), patches of an image, or a 3x3 convolution's
+// windows with at least a k-step of channels in whole 16-byte chunks (split
+// planes only where a k-step stays inside one tap). A staged row's byte
+// offsets are 32-bit.
 __host__ inline bool gemm_wave_fits(const GemmArgs &a, Math m) {
     const uint32_t epc = m == Math::F16 ? 8 : 4;
-    if (a.n % 8 != 0 || a.ksplit > 1 || a.ln_stats || a.flash_ops || a.row0 >= a.row1) return false;
+    if (a.n % 8 != 0 || a.ksplit > 1 || a.row0 >= a.row1) return false;
+    if (a.ln_stats && (a.load != 0 || a.bias || (m == Math::F16) != !a.ln_cb || a.k != 32 * a.ln_blocks || a.ln_blocks > 32 || a.ln_blocks % 2 != 0)) return false;
+    if (a.flash_ops && (a.load != 0 || m == Math::F32 || a.n % 192 != 0 || a.row0 % 16 != 0)) return false;
     if (a.load == 0) return a.k % 64 == 0 && a.k_pad == a.k && (uint64_t)a.m * a.k * 4 < (1ull << 31);
     if (a.load == 2) return a.k >= 32;
     if (a.load != 3 || a.p2 < 32 || a.p2 % epc != 0) return false;

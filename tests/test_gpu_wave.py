@@ -17,7 +17,7 @@ import pytest
 
 import oracle
 from beatlm_amd import hip, ir
-from tests.blockdata import CHAIN as H_, CHAIN_OUT as Y, chain, max_abs_err
+from tests.blockdata import CHAIN as H_, CHAIN_OUT as Y, block_values, block_weights, chain, max_abs_err
 
 pytestmark = pytest.mark.gpu
 
@@ -109,3 +109,49 @@ def test_a_wave_split_patch_embedding_matches_the_oracle(ctx, monkeypatch, gh, g
                                      oracle.uniform(43, cout, -0.1, 0.1))
     check(ctx, monkeypatch, {0: x, 1: w, 2: b}, [ir.op(ir.OP_PATCH_EMBED, [0, 1, 2], [gh, gw, p, cin, cout])],
           oracle.patch_embed(xf, wf, bf, gh, gw, p, cin, cout), math, tile, 1)
+
+
+@pytest.mark.parametrize("t", [17, 64, 65, 257])
+@pytest.mark.parametrize("math", MATHS)
+@pytest.mark.parametrize("tile", TILES)
+def test_wave_split_products_of_a_block_match_the_oracle(ctx, monkeypatch, t, math, tile):
+    """Two encoder blocks with every product wave-split: the QKV projections
+    write the attention's operands (tokens that end inside a 16-token run) and,
+    with fc1, apply folded LayerNorms whose rows' common offset is ten times
+    their spread; the out-projections and fc2 leave row statistics."""
+    d, h, mlp, eps = 192, 3, 768, 1e-6
+    monkeypatch.setenv("BL_GEMM_WAVE", tile)
+    x = oracle.uniform(61, t * d, -2.0, 2.0) + np.float32(0.0 if math == "f16" else 20.0)
+    ws = [block_weights(d, mlp, seed, "reference") for seed in (100, 200)]
+    g = ir.Graph()
+    g.tensor(0, ir.INPUT, t * d)
+    a = g.vit_block(ir.VitDims(t, d, h, mlp, eps), 0, 100, ir.ACTIVATION)
+    b = g.vit_block(ir.VitDims(t, d, h, mlp, eps), a.output, a.next_id, ir.OUTPUT)
+    vals = block_values(a, x, ws[0]) | block_values(b, x, ws[1])
+    if math == "f16":
+        vals = {k: v.astype(np.float16) for k, v in vals.items()}
+    if math == "f32":
+        ctx.set_f32_math(hip.F32_MATH_MFMA_F32)
+    try:
+        prep = ir.prepare(ctx, g, dtype=hip.F16 if math == "f16" else hip.F32)
+        try:
+            labels = [prep.kernels.label(k) for k in range(len(prep.kernels))]
+            assert sum(TILES[tile] in lab for lab in labels) == 8 and sum("folded into" in lab for lab in labels) == 3, labels
+            for tid, v in vals.items():
+                prep.write(tid, v)
+            prep.run()
+            ctx.synchronize()
+            got = prep.read(b.output).astype(np.float32)
+        finally:
+            prep.close()
+    finally:
+        ctx.set_f32_math(hip.F32_MATH_SPLIT_BF16)
+    if math == "f16":
+        x, ws = x.astype(np.float16).astype(np.float32), [{k: v.astype(np.float16).astype(np.float32) for k, v in w.items()} for w in ws]
+    want = oracle.vit_block(oracle.vit_block(x, ws[0], t, h, 64, mlp, eps), ws[1], t, h, 64, mlp, eps)
+    if math == "f16":
+        err = max_abs_err(got, want)
+        assert err <= F16_TOL, f"{labels}: max abs error {err:.3e}"
+    else:
+        bad = oracle.first_mismatch(got, want)
+        assert bad is None, f"{labels}: element {bad[0]} is {bad[1]}, the oracle says {bad[2]}"
