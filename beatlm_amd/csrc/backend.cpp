@@ -365,8 +365,9 @@ struct Launch {
     // statistics from x when the producer has not written them since x changed.
     int fold = -1;
     int fold_role = 0;
-    // A class-token prepend fused into the patch embedding before it: it
-    // launches nothing (the product writes its output).
+    // Launches nothing: a class-token prepend fused into the patch embedding
+    // before it, or a token-to-map into the LayerNorm before it, which write
+    // its output.
     bool fused = false;
 };
 enum FoldRole : int { FOLD_NONE = 0, FOLD_LAYER_NORM = 1, FOLD_CONSUMER = 2, FOLD_PRODUCER = 3 };
@@ -814,6 +815,79 @@ void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint3
         }
         ks->kernels[qi].label += " > fused into " + std::to_string(pi);
         ks->kernels[pi].label += " < prepend " + std::to_string(qi);
+    }
+}
+
+// An internal tensor's uses: its one writer and one reader among the kernels
+// (-1: none or several), the reader through binding `read_binding` alone.
+struct OneUse {
+    int writer = -1, reader = -1;
+    uint32_t read_binding = 0;
+};
+OneUse one_use(const bl_spec *specs, uint32_t n, uint32_t tensor) {
+    OneUse u;
+    int writers = 0, readers = 0;
+    for (uint32_t ki = 0; ki < n; ki++) {
+        const bl_spec &s = specs[ki];
+        const uint32_t last = s.n_bindings - 1;
+        if (s.bindings[last].tensor == tensor) {
+            writers++;
+            u.writer = (int)ki;
+        }
+        for (uint32_t b = 0; b < last; b++)
+            if (s.bindings[b].tensor == tensor) {
+                readers++;
+                u.reader = (int)ki;
+                u.read_binding = b;
+            }
+    }
+    if (writers != 1) u.writer = -1;
+    if (readers != 1) u.reader = -1;
+    return u;
+}
+
+// A LayerNorm whose output only the token-to-map right after it reads (the
+// encoder's taps): the LayerNorm writes rows 1 .. of its output as the map,
+// and the map launches nothing. Both whole, neither with an epilogue, and the
+// map's bytes apart from what the LayerNorm reads.
+void plan_maps(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t *internal, uint32_t n_internal) {
+    if (!n_internal || getenv("BL_NO_MAP_FUSION")) return;
+    std::vector<uint32_t> ids(internal, internal + n_internal);
+    std::sort(ids.begin(), ids.end());
+    for (uint32_t qi = 1; qi < n; qi++) {
+        const uint32_t li = qi - 1;
+        const bl_spec &qs = specs[qi], &ls = specs[li];
+        if (qs.main != BL_MAIN_TOKENS_TO_MAP || qs.part.count != 1 || qs.n_epilogue || ls.main != BL_MAIN_LAYER_NORM ||
+            ls.part.count != 1 || ls.n_epilogue)
+            continue;
+        const uint32_t t = ls.bindings[ls.n_bindings - 1].tensor;
+        const OneUse u = one_use(specs, n, t);
+        if (!std::binary_search(ids.begin(), ids.end(), t) || u.writer != (int)li || u.reader != (int)qi ||
+            u.read_binding != qs.reads[0] || qs.dims[2] != ls.dims[1] || ls.dims[0] != qs.dims[0] * qs.dims[1] + 1)
+            continue;
+        bool ok = true;
+        for (uint32_t si = 0; si < ks->sets && ok; si++) {
+            const Launch &L = ks->kernels[li].per_set[si], &Q = ks->kernels[qi].per_set[si];
+            const uint64_t esz = L.f16 ? 2 : 4;
+            auto apart = [&](const void *p, uint64_t elements) {
+                return (const char *)p >= Q.out_hi || (const char *)p + elements * esz <= Q.out_lo;
+            };
+            ok = L.family == Family::LAYER_NORM && L.fold < 0 && Q.family == Family::ELEMENT && (const void *)Q.el.a == L.ln.y &&
+                 (L.ln.channels * esz) % 16 == 0 && apart(L.ln.x, (uint64_t)L.ln.rows * L.ln.channels) &&
+                 apart(L.ln.gamma, L.ln.channels) && apart(L.ln.beta, L.ln.channels);
+        }
+        if (!ok) continue;
+        for (uint32_t si = 0; si < ks->sets; si++) {
+            Launch &L = ks->kernels[li].per_set[si], &Q = ks->kernels[qi].per_set[si];
+            L.ln.y = (char *)Q.el.y - (uint64_t)L.ln.channels * (L.f16 ? 2 : 4);
+            L.ln.row0 = 1;
+            L.out_lo = Q.out_lo;
+            L.out_hi = Q.out_hi;
+            Q.fused = true;
+            Q.out_lo = Q.out_hi = nullptr;
+        }
+        ks->kernels[li].label += " > map " + std::to_string(qi);
+        ks->kernels[qi].label += " > fused into " + std::to_string(li);
     }
 }
 
@@ -1689,6 +1763,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     }
     plan_prepends(ks, specs, n, internal, n_internal);
     plan_folds(ks, specs, n, sets, n_sets, internal, n_internal);
+    plan_maps(ks, specs, n, internal, n_internal);
     plan_waves(ks, ctx->compute_units);
     split_users.erase(std::remove_if(split_users.begin(), split_users.end(),
                                      [&](const std::pair<size_t, size_t> &u) { return ks->kernels[u.first].per_set[u.second].gemm.ksplit <= 1; }),
@@ -1995,7 +2070,7 @@ static hipError_t refresh_pack(bl_kernels *k, const Launch &L, hipStream_t s) {
 }
 
 static hipError_t launch(const Launch &L, hipStream_t s) {
-    if (L.fused) return hipSuccess;  // the product before it does its work
+    if (L.fused) return hipSuccess;  // the kernel beside it does its work
     switch (L.family) {
     case Family::LAYER_NORM: return L.fold_role == FOLD_LAYER_NORM ? hipSuccess : launch_layernorm(L.ln, L.f16, s);
     case Family::GEMM: {
