@@ -891,6 +891,54 @@ void plan_maps(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
     }
 }
 
+// A product with one output column right after the direct convolution whose
+// channels it reads (the depth head's last two convolutions): the convolution
+// adds up each pixel's channels in its epilogue and the product launches
+// nothing. Both whole, the channels (one block of the convolution's) an
+// internal tensor that nothing else reads, and the product's output apart from
+// the convolution's image. The channels' round trip through memory goes too: 34
+// MB at 518 x 518 in f32, the decoder 385 -> 379 us, in f16 286 -> 279.
+void plan_dots(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t *internal, uint32_t n_internal) {
+    if (!n_internal || getenv("BL_NO_DOT_FUSION")) return;
+    std::vector<uint32_t> ids(internal, internal + n_internal);
+    std::sort(ids.begin(), ids.end());
+    for (uint32_t qi = 1; qi < n; qi++) {
+        const uint32_t pi = qi - 1;
+        const bl_spec &qs = specs[qi], &ps = specs[pi];
+        if (qs.main != BL_MAIN_MATMUL || qs.part.count != 1 || ps.main != BL_MAIN_CONV3X3 || ps.part.count != 1) continue;
+        const uint32_t t = ps.bindings[ps.n_bindings - 1].tensor;
+        const OneUse u = one_use(specs, n, t);
+        if (!std::binary_search(ids.begin(), ids.end(), t) || u.writer != (int)pi || u.reader != (int)qi || u.read_binding != qs.reads[0])
+            continue;
+        bool ok = true;
+        for (uint32_t si = 0; si < ks->sets && ok; si++) {
+            const Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
+            const uint64_t image = (uint64_t)P.gemm.p0 * P.gemm.p1 * P.gemm.p2 * (P.f16 ? 2 : 4);
+            ok = P.family == Family::GEMM && P.tile == TILE_CONV3 && P.gemm.n == CD_NB && !P.gemm.c_planes && Q.family == Family::GEMV &&
+                 Q.gv.n == 1 && Q.gv.k == CD_NB && Q.gv.a == P.gemm.c && Q.gv.row0 == 0 && Q.gv.row1 == P.gemm.m && Q.f16 == P.f16 &&
+                 (Q.out_hi <= (const char *)P.gemm.a || (const char *)P.gemm.a + image <= Q.out_lo);
+            for (int e = 0; e < P.gemm.epi.n && ok; e++)
+                if (P.gemm.epi.kind[e] == BL_EPI_ADD)
+                    ok = Q.out_hi <= (const char *)P.gemm.epi.operand[e] ||
+                         (const char *)P.gemm.epi.operand[e] + (P.out_hi - P.out_lo) <= Q.out_lo;
+        }
+        if (!ok) continue;
+        for (uint32_t si = 0; si < ks->sets; si++) {
+            Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
+            P.gemm.dot_w = Q.gv.b;
+            P.gemm.dot_bias = Q.gv.bias;
+            P.gemm.dot_out = Q.gv.c;
+            P.gemm.dot_epi = Q.gv.epi;
+            P.out_lo = Q.out_lo;
+            P.out_hi = Q.out_hi;
+            Q.fused = true;
+            Q.out_lo = Q.out_hi = nullptr;
+        }
+        ks->kernels[qi].label += " > fused into " + std::to_string(pi);
+        ks->kernels[pi].label += " < product " + std::to_string(qi);
+    }
+}
+
 // LayerNorms folded into the products that read them. A LayerNorm L (no
 // epilogue, whole) over x [rows][D] whose output n is internal and read by
 // nothing but one later product G, as G's A (G whole, the ring kernel, plain
@@ -1764,6 +1812,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     plan_prepends(ks, specs, n, internal, n_internal);
     plan_folds(ks, specs, n, sets, n_sets, internal, n_internal);
     plan_maps(ks, specs, n, internal, n_internal);
+    plan_dots(ks, specs, n, internal, n_internal);
     plan_waves(ks, ctx->compute_units);
     split_users.erase(std::remove_if(split_users.begin(), split_users.end(),
                                      [&](const std::pair<size_t, size_t> &u) { return ks->kernels[u.first].per_set[u.second].gemm.ksplit <= 1; }),

@@ -117,6 +117,14 @@ struct GemmArgs {
     float *cls_ln_out;
     void *cls_shadow;
     EpilogueArgs cls_epi;
+    // A product with one output column fused into the direct 3x3 convolution
+    // whose CD_NB channels it reads (the depth head's last 1x1 convolution): a
+    // pixel's channels, through the epilogue and rounded to storage, times
+    // dot_w plus dot_bias (may be null), then dot_epi, at dot_out [m]; c is not
+    // written. Null dot_out: none.
+    const void *dot_w, *dot_bias;
+    void *dot_out;
+    EpilogueArgs dot_epi;
 };
 
 hipError_t launch_gemm_reduce(const GemmArgs &a, bool f16, hipStream_t s);
