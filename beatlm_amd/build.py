@@ -39,6 +39,7 @@ SOURCES = [
     "k_gemm_split.hip",
     "k_gemm_f16.hip",
     "k_wave.hip",
+    "k_point.hip",
     "k_flash.hip",
     "k_misc.hip",
     "static_attention.hip",

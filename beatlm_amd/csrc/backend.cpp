@@ -350,6 +350,9 @@ struct Launch {
     Dpt dpt = Dpt::RESIZE;
     DptArgs dp;
     GemvArgs gv;
+    // A short product (k_point.hip) in place of the family's own kernel.
+    bool point = false;
+    PointArgs pt;
     // The output's bytes (what the launch writes, the scratch aside).
     const char *out_lo = nullptr, *out_hi = nullptr;
     // A flash kernel whose QKV projections write its K and Vt (fl.prepped):
@@ -402,6 +405,7 @@ struct Pack {
     uint64_t vec_offset = 0;
     bool used = false;
     bool frag = false;  // fragment-major (packed_at): every reader takes B in registers
+    uint32_t tap_cols = 0;  // a transposed convolution's weights (PackArgs)
     bool folded() const { return gamma.ptr != nullptr; }
     bool reads(uint32_t a, uint64_t off, uint64_t bytes) const {
         auto hit = [&](uint32_t ar, uint64_t o, uint64_t sz) { return sz && ar == a && off < o + sz && o < off + bytes; };
@@ -891,6 +895,95 @@ void plan_maps(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
     }
 }
 
+// A bilinear resampling whose output only the 1x1 convolution right after it
+// reads (the fusion stages): the product blends the corners as it loads A
+// (k_point.hip) and the resampling launches nothing. Both whole, the
+// resampling with no epilogue. The product then reads the resampling's input
+// while it writes its own output, which a plan may place over it: such an
+// input, when the host never touches it, one product writes it and nothing
+// else reads it, moves to the kernels' workspace (Moved). Measured over whole
+// decoders (us, two launches -> one, bit for bit the same): 37 x 37 tokens f32
+// 398 -> 379, f16 294 -> 278; 19 x 19 f32 276 -> 268; 7 x 7 even.
+struct Moved {
+    uint32_t writer, reader;
+    uint64_t bytes;
+};
+void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t *internal, uint32_t n_internal,
+                  std::vector<Moved> &moved) {
+    if (!n_internal || getenv("BL_NO_RESIZE_FUSION")) return;
+    std::vector<uint32_t> ids(internal, internal + n_internal);
+    std::sort(ids.begin(), ids.end());
+    auto is_internal = [&](uint32_t t) { return std::binary_search(ids.begin(), ids.end(), t); };
+    for (uint32_t pi = 1; pi < n; pi++) {
+        const uint32_t qi = pi - 1;
+        const bl_spec &ps = specs[pi], &qs = specs[qi];
+        if (ps.main != BL_MAIN_MATMUL || ps.part.count != 1 || qs.main != BL_MAIN_RESIZE_BILINEAR || qs.part.count != 1 || qs.n_epilogue)
+            continue;
+        const uint32_t t = qs.bindings[qs.n_bindings - 1].tensor, xt = qs.bindings[qs.reads[0]].tensor;
+        const OneUse u = one_use(specs, n, t), ux = one_use(specs, n, xt);
+        if (!is_internal(t) || u.writer != (int)qi || u.reader != (int)pi || u.read_binding != ps.reads[0]) continue;
+        bool ok = true, move = false;
+        std::vector<PointArgs> args(ks->sets);
+        for (uint32_t si = 0; si < ks->sets && ok; si++) {
+            const Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
+            if (P.family != Family::GEMM || P.fold >= 0 || P.gemm.load != 0 || P.gemm.ksplit > 1 || Q.fused) {
+                ok = false;
+                break;
+            }
+            PointArgs &pa = args[si];
+            pa = PointArgs{};
+            pa.x = Q.dp.x;
+            pa.bias = P.gemm.bias;
+            pa.y = P.gemm.c;
+            pa.rows = P.gemm.m;
+            pa.n = P.gemm.n;
+            pa.k = P.gemm.k;
+            pa.ih = Q.dp.d[0];
+            pa.iw = Q.dp.d[1];
+            pa.ow = Q.dp.d[3];
+            pa.ry = Q.dp.ry;
+            pa.rx = Q.dp.rx;
+            pa.epi = P.gemm.epi;
+            pa.k_pad = P.gemm.k_pad;
+            pa.n_pad = P.gemm.n_pad;
+            const uint64_t x_bytes = (uint64_t)pa.ih * pa.iw * pa.k * (P.f16 ? 2 : 4);
+            ok = point_fits(pa) && P.gemm.a == Q.dp.y && pa.k == Q.dp.d[4] && pa.rows == Q.dp.d[2] * Q.dp.d[3];
+            if (P.out_lo < (const char *)pa.x + x_bytes && (const char *)pa.x < P.out_hi) move = true;
+        }
+        if (ok && move) {
+            ok = is_internal(xt) && ux.reader == (int)qi && ux.writer >= 0 && ux.writer < (int)qi && specs[ux.writer].part.count == 1;
+            for (uint32_t si = 0; si < ks->sets && ok; si++) {
+                const Launch &W = ks->kernels[ux.writer].per_set[si];
+                ok = W.family == Family::GEMM && !W.point && W.fold < 0 && !W.gemm.cls_out && !W.gemm.flash_ops && W.gemm.c == args[si].x;
+            }
+        }
+        if (!ok) continue;
+        if (move) moved.push_back({(uint32_t)ux.writer, pi, qs.bindings[qs.reads[0]].size});
+        for (uint32_t si = 0; si < ks->sets; si++) {
+            Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
+            P.point = true;
+            P.pt = args[si];
+            // A pack of its own (fragment-major, whatever the weights' other readers take).
+            Pack pk = ks->packs[P.pack];
+            pk.frag = true;
+            int found = -1;
+            for (size_t q = 0; q < ks->packs.size(); q++)
+                if (ks->packs[q].frag && !ks->packs[q].folded() && !ks->packs[q].tap_cols && ks->packs[q].math == pk.math &&
+                    ks->packs[q].arena == pk.arena && ks->packs[q].offset == pk.offset && ks->packs[q].k == pk.k && ks->packs[q].n == pk.n)
+                    found = (int)q;
+            if (found < 0) {
+                ks->packs.push_back(pk);
+                found = (int)ks->packs.size() - 1;
+            }
+            P.pack = found;
+            Q.fused = true;
+            Q.out_lo = Q.out_hi = nullptr;
+        }
+        ks->kernels[qi].label += " > fused into " + std::to_string(pi);
+        ks->kernels[pi].label += " < resize " + std::to_string(qi);
+    }
+}
+
 // A product with one output column right after the direct convolution whose
 // channels it reads (the depth head's last two convolutions): the convolution
 // adds up each pixel's channels in its epilogue and the product launches
@@ -1158,7 +1251,7 @@ void plan_waves(bl_kernels *ks, uint32_t compute_units) {
             int t = -1;
             GemmArgs g = L.gemm;
             g.ksplit = 1;
-            if (L.family == Family::GEMM && g.pipeline && L.tile != TILE_CONV3 && gemm_wave_fits(g, L.math))
+            if (L.family == Family::GEMM && !L.point && g.pipeline && L.tile != TILE_CONV3 && gemm_wave_fits(g, L.math))
                 t = wave_tile_of(g, L.math, compute_units, mode);
             if (si == 0) tile = t;
             else if (t != tile) tile = -1;
@@ -1169,7 +1262,7 @@ void plan_waves(bl_kernels *ks, uint32_t compute_units) {
     std::vector<uint8_t> ring(ks->packs.size(), 0);
     for (size_t ki = 0; ki < ks->kernels.size(); ki++)
         for (const Launch &L : ks->kernels[ki].per_set)
-            if (L.pack >= 0 && tiles[ki] < 0) ring[L.pack] = 1;
+            if (L.pack >= 0 && tiles[ki] < 0 && !L.point) ring[L.pack] = 1;
     for (bool again = true; again;) {
         again = false;
         for (size_t ki = 0; ki < ks->kernels.size(); ki++)
@@ -1516,7 +1609,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                 int pack = -1;
                 for (size_t q = 0; q < ks->packs.size(); q++) {
                     const Pack &pk = ks->packs[q];
-                    if (pk.arena == barena && pk.offset == boff && pk.math == fmath && pk.k == gk && pk.n == gn) pack = (int)q;
+                    if (pk.arena == barena && pk.offset == boff && pk.math == fmath && pk.k == gk && pk.n == gn && !pk.tap_cols) pack = (int)q;
                 }
                 if (pack < 0) {
                     Pack pk{};
@@ -1761,6 +1854,55 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                 L.dp.end = (uint64_t)pt.end * sh.per_unit;
                 L.dp.epi = epi;
                 variant = "per-element";
+                if (ct && pt.count == 1 && !getenv("BL_NO_POINT")) {
+                    // A whole transposed convolution of few channels: a product
+                    // over the input pixels (k_point.hip), in f32 on the matrix
+                    // cores for f32 storage as the vector ALUs had it (us over 37 x
+                    // 37 pixels, f32 and f16: 48 -> 48 with f = 4 11.9 -> 5.9 and
+                    // 11.6 -> 3.6, 96 -> 96 with f = 2 13.2 -> 5.3 and 13.0 ->
+                    // 3.8; over 7 x 7 in f32 4.8 -> 4.4 and 6.7 -> 5.2). More
+                    // channels than three slices stay on the vector ALUs.
+                    PointArgs pa{};
+                    pa.x = rd(0);
+                    pa.bias = L.dp.bias;
+                    pa.y = out_ptr;
+                    pa.rows = (uint32_t)std::min<uint64_t>((uint64_t)d[0] * d[1], UINT32_MAX);
+                    pa.k = d[2];
+                    pa.cout = d[3];
+                    pa.f = d[4];
+                    pa.n = (uint32_t)std::min<uint64_t>((uint64_t)d[4] * d[4] * d[3], UINT32_MAX - 128);
+                    pa.width = d[1];
+                    pa.k_pad = (pa.k + PACK_K - 1) / PACK_K * PACK_K;
+                    pa.n_pad = (pa.n + PACK_N - 1) / PACK_N * PACK_N;
+                    pa.epi = epi;
+                    if (d[4] < 256 && point_fits(pa)) {
+                        const bl_binding bb = resolve(s, s.reads[1], sets[si]);
+                        Pack pk{};
+                        pk.math = f16 ? Math::F16 : Math::F32;
+                        pk.src = rd(1);
+                        pk.arena = bb.arena;
+                        pk.offset = bb.offset;
+                        pk.size = bb.size;
+                        pk.k = pa.k;
+                        pk.n = pa.n;
+                        pk.k_pad = pa.k_pad;
+                        pk.n_pad = pa.n_pad;
+                        pk.tap_cols = pa.cout;
+                        for (size_t q = 0; q < ks->packs.size() && L.pack < 0; q++) {
+                            const Pack &o = ks->packs[q];
+                            if (o.arena == pk.arena && o.offset == pk.offset && o.math == pk.math && o.k == pk.k && o.n == pk.n &&
+                                o.tap_cols == pk.tap_cols)
+                                L.pack = (int)q;
+                        }
+                        if (L.pack < 0) {
+                            ks->packs.push_back(pk);
+                            L.pack = (int)ks->packs.size() - 1;
+                        }
+                        L.point = true;
+                        L.pt = pa;
+                        variant = f16 ? "mfma-f16 rows" : "mfma-f32 rows";
+                    }
+                }
                 break;
             }
             case BL_MAIN_FLASH_ATTENTION: {
@@ -1812,6 +1954,8 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     plan_prepends(ks, specs, n, internal, n_internal);
     plan_folds(ks, specs, n, sets, n_sets, internal, n_internal);
     plan_maps(ks, specs, n, internal, n_internal);
+    std::vector<Moved> moved;
+    plan_resizes(ks, specs, n, internal, n_internal, moved);
     plan_dots(ks, specs, n, internal, n_internal);
     plan_waves(ks, ctx->compute_units);
     split_users.erase(std::remove_if(split_users.begin(), split_users.end(),
@@ -1848,7 +1992,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                               g.k % 64 == 0 && g.k >= 64 && g.k_pad == g.k && (L.tile == TILE_32x64 || L.tile == TILE_64x64) &&
                               (breg_mode == 1 || (g.k >= 2 * g.n && g.k / 64 >= 12));
                 int &v = all[L.pack];
-                const bool frag = wave || L.gemm.breg;
+                const bool frag = wave || L.gemm.breg || L.point;
                 v = v < 0 ? (int)frag : (v && frag);
             }
         for (size_t q = 0; q < ks->packs.size(); q++) ks->packs[q].frag = all[q] == 1;
@@ -1910,6 +2054,9 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
         for (uint32_t si = 0; si < ks->sets; si++)
             items.push_back({align256(fold_stats_bytes(f)) + align256(fold_plane_bytes(f, ks->kernels[f.consumer].per_set[si])),
                              f.producer, f.consumer, (int)si, 0});
+    const size_t moved_item = items.size();
+    for (const Moved &mv : moved)
+        for (uint32_t si = 0; si < ks->sets; si++) items.push_back({align256(mv.bytes), mv.writer, mv.reader, (int)si, 0});
     const uint64_t workspace = place_workspace(items);
     if (workspace) {
         ks->workspace = (char *)bl_device_alloc(ctx, workspace);
@@ -1938,6 +2085,18 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
         for (size_t e = 0; e < ks->fold_alias.size(); e++)
             if (overlap(item, fold_item + e)) ks->kernel_clobbers[ki].push_back((uint32_t)e);
     }
+    // A moved tensor's writer overwrites the folds that share its bytes too.
+    for (size_t q = 0; q < moved.size(); q++)
+        for (uint32_t si = 0; si < ks->sets; si++) {
+            const size_t item = moved_item + q * ks->sets + si;
+            Launch &W = ks->kernels[moved[q].writer].per_set[si], &P = ks->kernels[moved[q].reader].per_set[si];
+            W.gemm.c = ks->workspace + items[item].at;
+            W.out_lo = (const char *)W.gemm.c;
+            W.out_hi = W.out_lo + moved[q].bytes;
+            P.pt.x = W.gemm.c;
+            for (size_t e = 0; e < ks->fold_alias.size(); e++)
+                if (overlap(item, fold_item + e)) ks->kernel_clobbers[moved[q].writer].push_back((uint32_t)e);
+        }
     for (size_t e = 0; e < ks->fold_alias.size(); e++)
         for (size_t g = 0; g < ks->fold_alias.size(); g++)
             if (g != e && overlap(fold_item + e, fold_item + g)) ks->fold_alias[e].push_back((uint32_t)g);
@@ -2109,7 +2268,7 @@ static hipError_t refresh_pack(bl_kernels *k, const Launch &L, hipStream_t s) {
     if (!pk.dynamic && !pk.stale) return hipSuccess;
     PackArgs pa{pk.src, (char *)k->pack_buffer + pk.dst_offset, pk.k, pk.n, pk.k_pad, pk.n_pad,
                 pk.gamma.ptr, pk.beta.ptr, pk.bias.ptr,
-                pk.folded() ? (float *)((char *)k->pack_buffer + pk.vec_offset) : nullptr, pk.frag ? 1u : 0u};
+                pk.folded() ? (float *)((char *)k->pack_buffer + pk.vec_offset) : nullptr, pk.frag ? 1u : 0u, pk.tap_cols};
     hipError_t e = launch_pack(pa, pk.math, s);
     if (e == hipSuccess) {
         pk.stale = false;
@@ -2120,6 +2279,12 @@ static hipError_t refresh_pack(bl_kernels *k, const Launch &L, hipStream_t s) {
 
 static hipError_t launch(const Launch &L, hipStream_t s) {
     if (L.fused) return hipSuccess;  // the kernel beside it does its work
+    if (L.point) {
+        PointArgs pa = L.pt;
+        pa.b = L.gemm.b;
+        if (L.family == Family::GEMM) pa.y_planes = L.gemm.c_planes;
+        return launch_point(pa, L.math, s);
+    }
     switch (L.family) {
     case Family::LAYER_NORM: return L.fold_role == FOLD_LAYER_NORM ? hipSuccess : launch_layernorm(L.ln, L.f16, s);
     case Family::GEMM: {

@@ -141,6 +141,9 @@ struct PackArgs {
     const void *gamma, *beta, *bias;
     float *vec;
     uint32_t frag;  // pack fragment-major (packed_at) for the B-in-registers kernel
+    // A transposed convolution's weights [f f][k][tap_cols] as a product's B:
+    // column n is (tap n / tap_cols, channel n % tap_cols). 0: B [k][n].
+    uint32_t tap_cols;
 };
 
 // Where element (n, k) of a packed B plane lies. Row layout: [n_pad][k_pad].
@@ -254,6 +257,32 @@ struct DptArgs {
     uint64_t start, end;  // output elements of the part
     EpilogueArgs epi;
 };
+
+// A short product over many rows (k_point.hip): y = A w + bias, then the
+// epilogue, where A is x's rows (a transposed convolution with kernel = stride
+// = f: y's element (pixel, tap, channel) scattered to its output pixel, n = f f
+// cout) or a bilinear resampling with aligned corners
+// of the image x [ih][iw][k] to rows of ow pixels (ih > 0).
+struct PointArgs {
+    const void *x, *bias;
+    const void *b;            // packed fragment-major
+    void *y;
+    uint32_t rows, n, k;
+    uint32_t k_pad, n_pad;
+    uint32_t f, width, cout;  // the transposed convolution's factor (0: none), input width, channels
+    uint32_t ih, iw, ow;      // the resampling's image and output width
+    float ry, rx;             // input rows (columns) per output row (column)
+    uint64_t y_planes;        // y kept as hi and lo bf16 planes this many elements apart (0: as stored)
+    EpilogueArgs epi;
+};
+// Vectors of 8 in and out, k of at most three 32-wide slices, 32-bit rows.
+__host__ inline bool point_fits(const PointArgs &a) {
+    return a.k % 8 == 0 && a.k >= 8 && a.k <= 96 && a.n % 8 == 0 && a.n >= 8 && a.n <= (1u << 16) && a.rows > 0 &&
+           a.rows < (1u << 30) && a.k_pad % 32 == 0 && a.k_pad >= a.k && a.n_pad % 128 == 0 && a.n_pad >= a.n && (a.f ? a.cout % 8 == 0 && a.f < 256 && a.n == a.f * a.f * a.cout && !a.ih : a.ih > 0) &&
+           (uint64_t)a.rows * (a.f ? a.f * a.f : 1) < (1ull << 31);
+}
+constexpr uint32_t POINT_GROUPS = 1024;
+hipError_t launch_point(const PointArgs &a, Math m, hipStream_t s);
 
 // One element per invocation: the standalone map, the token copies.
 enum class PerElement : int { MAP = 0, PREPEND = 1, DROP_FIRST = 2 };

@@ -56,6 +56,33 @@ def check(ctx, arrays, ops, oracle_of, math, marks):
         assert bad is None, f"{labels}: element {bad[0]} is {bad[1]}, the oracle says {bad[2]}"
 
 
+@pytest.mark.parametrize("h,w,cin,cout,f", [(1, 1, 8, 8, 2), (3, 5, 48, 48, 4), (4, 4, 96, 24, 2), (7, 9, 40, 16, 3), (37, 37, 32, 8, 1)])
+@pytest.mark.parametrize("math", MATHS)
+def test_a_transposed_convolution_as_a_product_matches_the_oracle(ctx, h, w, cin, cout, f, math):
+    arrays = [oracle.uniform(1 + cin, h * w * cin, -2.0, 2.0), oracle.fan_in_weights(2 + cout, f * f * cin * cout, cin),
+              oracle.uniform(3, cout, -0.1, 0.1)]
+    check(ctx, arrays, [ir.op(ir.OP_CONV_TRANSPOSE, [0, 1, 2], [h, w, cin, cout, f])],
+          lambda x, wt, b: oracle.conv_transpose(x, wt, b, h, w, cin, cout, f), math, ["rows"])
+
+
+@pytest.mark.parametrize("ih,iw,oh,ow,c,n", [(1, 1, 3, 2, 8, 8), (5, 7, 10, 14, 64, 64), (6, 4, 11, 9, 96, 72), (9, 9, 5, 4, 32, 136),
+                                             (3, 8, 1, 1, 40, 16)])
+@pytest.mark.parametrize("math", MATHS)
+def test_a_resampling_blended_into_its_product_matches_the_oracle(ctx, ih, iw, oh, ow, c, n, math):
+    """conv -> resize -> 1x1 -> relu: the convolution's output is the internal
+    tensor that may move."""
+    arrays = [oracle.uniform(11 + c, ih * iw * c, -2.0, 2.0), oracle.fan_in_weights(12, 9 * c * c, 9 * c), oracle.fan_in_weights(13 + n, c * n, c),
+              oracle.uniform(14, n, -0.1, 0.1)]
+    ops = [ir.op(ir.OP_CONV3X3, [0, 1, ir.NONE], [ih, iw, c, c, 1]), ir.op(ir.OP_RESIZE_BILINEAR, [H_], [ih, iw, oh, ow, c]),
+           ir.op(ir.OP_MATMUL, [H_ + 1, 2, 3], [oh * ow, c, n]), ir.op(ir.OP_RELU, [H_ + 2], [oh * ow * n])]
+
+    def want(x, wc, w, b):
+        y = oracle.resize_bilinear(oracle.conv3x3(x, wc, None, ih, iw, c, c, 1), ih, iw, oh, ow, c)
+        return np.maximum(oracle.matmul(y, w, b, oh * ow, c, n), 0)
+
+    check(ctx, arrays, ops, want, math, ["< resize 1", "fused into 2"])
+
+
 @pytest.mark.parametrize("h,w,cin", [(130, 255, 32), (67, 513, 40)])
 @pytest.mark.parametrize("math", ["bf16x3", "f16"])
 def test_a_convolution_that_adds_up_its_channels_matches_the_oracle(ctx, h, w, cin, math):
