@@ -811,7 +811,7 @@ void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint3
             g.epi_mode = 3;
             g.cls_token = Q.el.a;
             g.cls_out = Q.el.y;
-            g.cls_epi = Q.el.epi;
+            g.side_epi = Q.el.epi;
             P.out_lo = Q.out_lo;
             P.out_hi = Q.out_hi;
             Q.fused = true;
@@ -1021,7 +1021,7 @@ void plan_dots(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
             P.gemm.dot_w = Q.gv.b;
             P.gemm.dot_bias = Q.gv.bias;
             P.gemm.dot_out = Q.gv.c;
-            P.gemm.dot_epi = Q.gv.epi;
+            P.gemm.side_epi = Q.gv.epi;
             P.out_lo = Q.out_lo;
             P.out_hi = Q.out_hi;
             Q.fused = true;

@@ -109,22 +109,22 @@ struct GemmArgs {
     // the plain kernel): c is x's second row, so that the product's rows are
     // x's rows 1 .. m, and the epilogue's added tensors are read one row on
     // likewise; the workgroups of the first row band also write x's first
-    // row, cls_epi applied to cls_token [n], at cls_out (x itself), with its
+    // row, side_epi applied to cls_token [n], at cls_out (x itself), with its
     // block statistics at cls_ln_out and its planes at cls_shadow when the
     // product is a fold's producer. Null cls_out: none.
     const void *cls_token;
     void *cls_out;
     float *cls_ln_out;
     void *cls_shadow;
-    EpilogueArgs cls_epi;
     // A product with one output column fused into the direct 3x3 convolution
     // whose CD_NB channels it reads (the depth head's last 1x1 convolution): a
     // pixel's channels, through the epilogue and rounded to storage, times
-    // dot_w plus dot_bias (may be null), then dot_epi, at dot_out [m]; c is not
+    // dot_w plus dot_bias (may be null), then side_epi, at dot_out [m]; c is not
     // written. Null dot_out: none.
     const void *dot_w, *dot_bias;
     void *dot_out;
-    EpilogueArgs dot_epi;
+    // Of the fused prepend or the fused one-column product (never both).
+    EpilogueArgs side_epi;
 };
 
 hipError_t launch_gemm_reduce(const GemmArgs &a, bool f16, hipStream_t s);
