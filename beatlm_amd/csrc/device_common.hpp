@@ -43,14 +43,6 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// The sum over the LPR consecutive lanes that hold one row (LPR a power of 2).
-template <int LPR>
-__device__ __forceinline__ float row_sum(float v) {
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
-}
-
 // v plus v of the lane DPP control CTRL names (row and bank masks full).
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {

@@ -9,6 +9,18 @@
 namespace bl {
 namespace {
 
+// The sum over the LPR consecutive lanes that hold one row: DPP within 16
+// lanes and v_permlane32_swap across halves, no LDS round trip but the one
+// between the 16-lane rows of a half.
+template <int LPR>
+__device__ __forceinline__ float lanes_sum(float v) {
+    static_assert(LPR == 16 || LPR == 32 || LPR == 64, "rows of 16, 32 or 64 lanes");
+    v = row16_sum(v);
+    if constexpr (LPR >= 32) v += __shfl_xor(v, 16, WAVE);
+    if constexpr (LPR == 64) v = sum_xor32(v);
+    return v;
+}
+
 // ------------------------------------------------------------------------
 // Layer norm (MainOp::LayerNorm, kernel.rs:643-659; reference arithmetic
 // wgsl.rs:519-585): (x - mean) * rsqrt(var + eps) * gamma + beta per row,
@@ -27,20 +39,40 @@ __global__ __launch_bounds__(256) void layernorm_kernel(LayerNormArgs a) {
     if (row >= a.row1) return;
     const uint32_t C = a.channels, nch = C / VEC;
     const T *x = (const T *)a.x + (uint64_t)row * C;
+    // gamma and beta are loaded with the row: a load after the reductions
+    // would put one more round trip into the chain, which is what bounds a
+    // LayerNorm of a few thousand rows (us, with the DPP sums, before ->
+    // after: 1370 x 384 f32 3.35 -> 3.02, 1370 x 768 f16 3.28 -> 2.81, 1370 x
+    // 1024 f16 3.39 -> 3.24, 5477 x 384 f16 3.70 -> 3.35).
+    const T *gamma = (const T *)a.gamma, *beta = (const T *)a.beta;
     float v[NV][VEC];
+    V xv[NV], gv[NV], bv[NV];
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        uint32_t c = lane + 64 * i;
-        V chunk = {};
-        if (c < nch) chunk = *(const V *)(x + c * VEC);
+        const uint32_t c = lane + 64 * i;
+        xv[i] = gv[i] = bv[i] = V{};
+        if (c < nch) xv[i] = *(const V *)(x + c * VEC);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const uint32_t c = lane + 64 * i;
+        if (c < nch) {
+            gv[i] = *(const V *)(gamma + c * VEC);
+            bv[i] = *(const V *)(beta + c * VEC);
+        }
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const V chunk = xv[i];
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
             v[i][e] = to_f32(chunk[e]);
             sum += v[i][e];
         }
     }
-    const float mean = wave_sum(sum) / (float)C;
+    const float mean = lanes_sum<64>(sum) / (float)C;
     float sq = 0.0f;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
@@ -52,18 +84,16 @@ __global__ __launch_bounds__(256) void layernorm_kernel(LayerNormArgs a) {
             }
         }
     }
-    const float inv = 1.0f / sqrtf(wave_sum(sq) / (float)C + a.eps);
-    const T *gamma = (const T *)a.gamma, *beta = (const T *)a.beta;
+    const float inv = 1.0f / sqrtf(lanes_sum<64>(sq) / (float)C + a.eps);
     T *y = (T *)a.y + (uint64_t)row * C;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         uint32_t c = lane + 64 * i;
         if (c >= nch) continue;
-        V gv = *(const V *)(gamma + c * VEC), bv = *(const V *)(beta + c * VEC);
         V out;
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
-            float r = (v[i][e] - mean) * inv * to_f32(gv[e]) + to_f32(bv[e]);
+            float r = (v[i][e] - mean) * inv * to_f32(gv[i][e]) + to_f32(bv[i][e]);
             if (a.epi.n) r = apply_epilogue<T>(a.epi, r, (uint64_t)row * C + c * VEC + e);
             out[e] = from_f32<T>(r);
         }
@@ -93,19 +123,31 @@ __global__ __launch_bounds__(256) void layernorm3_kernel(LayerNormArgs a) {
     const bool ok = row < a.row1;
     const uint32_t C = a.channels;
     const T *x = (const T *)a.x + (uint64_t)(ok ? row : a.row0) * C;
+    const T *gamma = (const T *)a.gamma, *beta = (const T *)a.beta;
     float v[3][VEC];
+    V xv[3], gv[3], bv[3];  // gamma and beta with the row, as above
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         const V *src = (const V *)(x + (l + LPR * i) * VEC);
-        const V chunk = NT ? __builtin_nontemporal_load(src) : *src;
+        xv[i] = NT ? __builtin_nontemporal_load(src) : *src;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        gv[i] = *(const V *)(gamma + (l + LPR * i) * VEC);
+        bv[i] = *(const V *)(beta + (l + LPR * i) * VEC);
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const V chunk = xv[i];
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
             v[i][e] = to_f32(chunk[e]);
             sum += v[i][e];
         }
     }
-    const float mean = row_sum<LPR>(sum) / (float)C;
+    const float mean = lanes_sum<LPR>(sum) / (float)C;
     float sq = 0.0f;
 #pragma unroll
     for (int i = 0; i < 3; i++)
@@ -114,18 +156,16 @@ __global__ __launch_bounds__(256) void layernorm3_kernel(LayerNormArgs a) {
             const float d = v[i][e] - mean;
             sq += d * d;
         }
-    const float inv = 1.0f / sqrtf(row_sum<LPR>(sq) / (float)C + a.eps);
+    const float inv = 1.0f / sqrtf(lanes_sum<LPR>(sq) / (float)C + a.eps);
     if (!ok) return;
-    const T *gamma = (const T *)a.gamma, *beta = (const T *)a.beta;
     T *y = (T *)a.y + (uint64_t)row * C;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         const uint32_t c = l + LPR * i;
-        const V gv = *(const V *)(gamma + c * VEC), bv = *(const V *)(beta + c * VEC);
         V out;
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
-            float r = (v[i][e] - mean) * inv * to_f32(gv[e]) + to_f32(bv[e]);
+            float r = (v[i][e] - mean) * inv * to_f32(gv[i][e]) + to_f32(bv[i][e]);
             if (a.epi.n) r = apply_epilogue<T>(a.epi, r, (uint64_t)row * C + c * VEC + e);
             out[e] = from_f32<T>(r);
         }
