@@ -926,7 +926,13 @@ void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32
         std::vector<PointArgs> args(ks->sets);
         for (uint32_t si = 0; si < ks->sets && ok; si++) {
             const Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
-            if (P.family != Family::GEMM || P.fold >= 0 || P.gemm.load != 0 || P.gemm.ksplit > 1 || Q.fused) {
+            // An attention's K and Vt come from the projection's own kernels,
+            // which this one is none of.
+            bool projection = false;
+            for (const Kernel &k : ks->kernels)
+                if (k.per_set[si].family == Family::FLASH && k.per_set[si].fl.qkv == P.gemm.c) projection = true;
+            if (P.family != Family::GEMM || P.fold >= 0 || P.gemm.load != 0 || P.gemm.ksplit > 1 || Q.fused ||
+                (projection && P.math != Math::F32 && P.gemm.epi_mode == 0)) {
                 ok = false;
                 break;
             }
@@ -2125,7 +2131,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                     Launch &P = ks->kernels[j].per_set[si];
                     if (P.family == Family::FLASH && P.fl.qkv == F.fl.qkv) continue;
                     if (P.family != Family::GEMM || P.gemm.c != F.fl.qkv) break;
-                    if (P.gemm.load != 0 || P.gemm.epi_mode != 0 || P.gemm.ksplit > 1 || P.math != F.math || P.gemm.m != F.fl.tokens ||
+                    if (P.point || P.gemm.load != 0 || P.gemm.epi_mode != 0 || P.gemm.ksplit > 1 || P.math != F.math || P.gemm.m != F.fl.tokens ||
                         P.gemm.n != 3 * F.fl.heads * FLASH_HEAD_DIM)
                         ok = false;
                     producers.push_back(j);
@@ -2280,6 +2286,7 @@ static hipError_t refresh_pack(bl_kernels *k, const Launch &L, hipStream_t s) {
 static hipError_t launch(const Launch &L, hipStream_t s) {
     if (L.fused) return hipSuccess;  // the kernel beside it does its work
     if (L.point) {
+        if (L.gemm.flash_ops) return hipErrorInvalidValue;  // it writes no K or Vt
         PointArgs pa = L.pt;
         pa.b = L.gemm.b;
         if (L.family == Family::GEMM) pa.y_planes = L.gemm.c_planes;

@@ -1,0 +1,134 @@
+"""Plans of several kernels composed: launches that take two kernels' place
+next to other plans that read or write the same tensors, programs of several
+binding sets whose kernels interleave, parts that do not cover their tensor,
+and outputs the memory plan lays over what an earlier kernel still reads.
+
+Tolerance for f32 storage: |got - want| <= 1e-4 + 1e-4 |want|
+(reference.rs:22-24); for f16 storage, max abs error <= 2e-2 against the
+oracle on the same f16-rounded inputs.
+"""
+
+import numpy as np
+import pytest
+
+import oracle
+from beatlm_amd import hip, ir
+from tests.blockdata import max_abs_err
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-6
+F16_TOL = 2e-2
+MATHS = ["bf16x3", "f32", "f16"]
+STAND_IN = 1 << 18
+
+
+@pytest.fixture
+def math(ctx, request):
+    if request.param == "f32":
+        ctx.set_f32_math(hip.F32_MATH_MFMA_F32)
+    yield request.param
+    ctx.set_f32_math(hip.F32_MATH_SPLIT_BF16)
+
+
+def compare(got, want, math, what):
+    if math == "f16":
+        err = max_abs_err(got, want)
+        assert err <= F16_TOL, f"{what}: max abs error {err:.3e}"
+    else:
+        bad = oracle.first_mismatch(got, want)
+        assert bad is None, f"{what}: element {bad[0]} is {bad[1]}, the oracle says {bad[2]}"
+
+
+class Net:
+    """A graph from (operation, output role) pairs: tensor i of `inputs`
+    ((role, elements) each) is i, operation i writes 100 + i. Planned and
+    prepared through the C ABI; `change(specs)` may edit the specs, and every
+    tensor that is no weight gets stand-ins of its own in each set past the first."""
+
+    def __init__(self, ctx, inputs, ops, math, sets=1, change=None):
+        g = ir.Graph()
+        for i, (role, n) in enumerate(inputs):
+            g.tensor(i, role, n)
+        for i, (o, role) in enumerate(ops):
+            g.tensor(100 + i, role, ir.output_elements(o))
+            g.push(o, 100 + i)
+        self.program = g.lower().fuse_attention()
+        self.f16 = math == "f16"
+        self.program.set_dtype(hip.F16 if self.f16 else hip.F32)
+        tensors = self.program.tensors()
+        descs, own, last = list(tensors), [{t.id: t.id for t in tensors}], len(self.program) - 1
+        for s in range(1, sets):
+            own.append({})
+            for t in tensors:
+                if self.program.role(t.id) != ir.WEIGHT:
+                    own[s][t.id] = s * STAND_IN + t.id
+                    descs.append(ir.tensor_desc(own[s][t.id], t.dtype, t.elements, 0, last))
+        self.plan = ir.Plan(descs, ir.profile("mi355x"))
+        self.own, self.elements = own, {t.id: t.elements for t in tensors}
+        self.arenas = hip.Arenas(ctx, self.plan.arenas())
+        specs = self.program.specs(self.plan)
+        if change:
+            change(specs)
+        subs = None
+        if sets > 1:
+            subs = []
+            for mine in own:
+                at = {t: self.plan.placement(s) for t, s in mine.items() if t != s}
+                subs.append([hip.Substitution(t, mine[t], p.arena, 0, p.offset, p.size) for t, p in at.items()])
+        internal = [t.id for t in tensors if self.program.role(t.id) == ir.ACTIVATION]
+        self.kernels = hip.Kernels(ctx, self.arenas, specs, sets=subs, internal=internal)
+        self.labels = [self.kernels.label(k) for k in range(len(self.kernels))]
+        self.ctx = ctx
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *_):
+        self.kernels.close()
+        self.arenas.close()
+
+    def at(self, tid, s=0):
+        return self.plan.placement(self.own[s].get(tid, tid))
+
+    def write(self, tid, v, s=0):
+        p = self.at(tid, s)
+        self.arenas.write(p.arena, p.offset, np.ascontiguousarray(v, np.float16 if self.f16 else np.float32))
+
+    def read(self, tid, s=0):
+        p = self.at(tid, s)
+        return self.arenas.read(p.arena, p.offset, self.elements[tid], np.float16 if self.f16 else np.float32).astype(np.float32)
+
+    def overlap(self, a, b):
+        """Whether the plan lays tensors a and b over each other in set 0."""
+        p, q = self.at(a), self.at(b)
+        return p.arena == q.arena and p.offset < q.offset + q.size and q.offset < p.offset + p.size
+
+
+def stored(math, a):
+    """The values as stored, as the oracle reads them."""
+    return a.astype(np.float16).astype(np.float32) if math == "f16" else a
+
+
+@pytest.mark.parametrize("h,w,oh,ow,heads", [(4, 4, 8, 8, 1), (3, 5, 9, 7, 2)])
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+def test_attention_over_a_projection_of_a_resampling(ctx, h, w, oh, ow, heads, math):
+    """resize -> QKV projection -> attention: the attention's keys and values
+    are the projection's, whoever writes them."""
+    t, n = oh * ow, 3 * heads * 64
+    wq, bq = (stored(math, a) for a in (oracle.fan_in_weights(41, 64 * n, 64), oracle.uniform(42, n, -0.1, 0.1)))
+    ops = [(ir.op(ir.OP_RESIZE_BILINEAR, [0], [h, w, oh, ow, 64]), ir.ACTIVATION), (ir.op(ir.OP_MATMUL, [100, 1, 2], [t, 64, n]), ir.ACTIVATION),
+           (ir.op(ir.OP_ATTENTION_SCORES, [101], [t, heads, 64]), ir.ACTIVATION),
+           (ir.op(ir.OP_SCALE, [102], [t * heads * t], 0.125), ir.ACTIVATION), (ir.op(ir.OP_SOFTMAX, [103], [t * heads, t]), ir.ACTIVATION),
+           (ir.op(ir.OP_ATTENTION_VALUES, [104, 101], [t, heads, 64]), ir.OUTPUT)]
+    with Net(ctx, [(ir.INPUT, h * w * 64), (ir.WEIGHT, 64 * n), (ir.WEIGHT, n)], ops, math) as net:
+        assert "flash_attention" in net.labels[-1], net.labels
+        net.write(1, wq)
+        net.write(2, bq)
+        for seed in (43, 44):
+            x = stored(math, oracle.uniform(seed, h * w * 64, -2.0, 2.0))
+            net.write(0, x)
+            net.kernels.encode_all()
+            ctx.synchronize()
+            qkv = oracle.matmul(oracle.resize_bilinear(x, h, w, oh, ow, 64), wq, bq, t, 64, n)
+            compare(net.read(105), oracle.attention(qkv, t, heads, 64, 0.125), math, f"{net.labels}, input {seed}")
