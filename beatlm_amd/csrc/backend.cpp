@@ -964,7 +964,10 @@ void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32
             }
         }
         if (!ok) continue;
-        if (move) moved.push_back({(uint32_t)ux.writer, pi, qs.bindings[qs.reads[0]].size});
+        if (move) {
+            moved.push_back({(uint32_t)ux.writer, pi, qs.bindings[qs.reads[0]].size});
+            ks->kernels[ux.writer].label += " > workspace";
+        }
         for (uint32_t si = 0; si < ks->sets; si++) {
             Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
             P.point = true;
@@ -1355,13 +1358,14 @@ extern "C" int bl_kernels_create(bl_ctx *ctx, bl_arenas *arenas, const bl_spec *
 namespace {
 
 // One item of the backend's workspace: its bytes, the kernels from its first
-// writer to its last reader (inclusive), its binding set (-1: any), and its
-// offset once placed.
+// writer to its last reader (inclusive), its binding set (-1: any), its
+// offset once placed, and whether it shares bytes with no other item.
 struct WsItem {
     uint64_t size;
     uint32_t first, last;
     int set;
     uint64_t at;
+    bool alone = false;
 };
 
 // Places the items as the memory plan places tensors in an arena
@@ -1369,14 +1373,16 @@ struct WsItem {
 // lowest 256-byte aligned offset clear of every placed item it may be live
 // with. Items of two different binding sets are taken to be live together
 // (a frame loop may interleave the sets' ranges); otherwise two items are
-// live together when their kernel intervals overlap. Returns the bytes the
-// placement spans.
+// live together when their kernel intervals overlap. What shares bytes can be
+// made again (a fold's statistics) or lives for one launch (partial sums); an
+// item that cannot (a moved tensor) is live with every other. Returns the
+// bytes the placement spans.
 uint64_t place_workspace(std::vector<WsItem> &items) {
     std::vector<size_t> order(items.size());
     for (size_t i = 0; i < order.size(); i++) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return items[a].size > items[b].size; });
     auto together = [&](const WsItem &a, const WsItem &b) {
-        if (a.set >= 0 && b.set >= 0 && a.set != b.set) return true;
+        if (a.alone || b.alone || (a.set >= 0 && b.set >= 0 && a.set != b.set)) return true;
         return a.first <= b.last && b.first <= a.last;
     };
     std::vector<size_t> placed;
@@ -1971,7 +1977,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     // arenas, laid out by lifetime (place_workspace): the packed weights and
     // the attention scratch for the whole program, each split-k GEMM's
     // partial sums for its own launch, each folded LayerNorm's statistics and
-    // planes from its producer to its consumer.
+    // planes from its producer to its consumer, each moved tensor.
     auto align256 = [](uint64_t b) { return (b + 255) / 256 * 256; };
     // B in registers (GemmArgs::breg) for ring-kernel products of 64-column
     // tiles of at most 64 rows, one group of waves and 64-wide k-steps whose
@@ -2062,7 +2068,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                              f.producer, f.consumer, (int)si, 0});
     const size_t moved_item = items.size();
     for (const Moved &mv : moved)
-        for (uint32_t si = 0; si < ks->sets; si++) items.push_back({align256(mv.bytes), mv.writer, mv.reader, (int)si, 0});
+        for (uint32_t si = 0; si < ks->sets; si++) items.push_back({align256(mv.bytes), mv.writer, mv.reader, (int)si, 0, true});
     const uint64_t workspace = place_workspace(items);
     if (workspace) {
         ks->workspace = (char *)bl_device_alloc(ctx, workspace);
@@ -2091,17 +2097,13 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
         for (size_t e = 0; e < ks->fold_alias.size(); e++)
             if (overlap(item, fold_item + e)) ks->kernel_clobbers[ki].push_back((uint32_t)e);
     }
-    // A moved tensor's writer overwrites the folds that share its bytes too.
     for (size_t q = 0; q < moved.size(); q++)
         for (uint32_t si = 0; si < ks->sets; si++) {
-            const size_t item = moved_item + q * ks->sets + si;
             Launch &W = ks->kernels[moved[q].writer].per_set[si], &P = ks->kernels[moved[q].reader].per_set[si];
-            W.gemm.c = ks->workspace + items[item].at;
+            W.gemm.c = ks->workspace + items[moved_item + q * ks->sets + si].at;
             W.out_lo = (const char *)W.gemm.c;
             W.out_hi = W.out_lo + moved[q].bytes;
             P.pt.x = W.gemm.c;
-            for (size_t e = 0; e < ks->fold_alias.size(); e++)
-                if (overlap(item, fold_item + e)) ks->kernel_clobbers[moved[q].writer].push_back((uint32_t)e);
         }
     for (size_t e = 0; e < ks->fold_alias.size(); e++)
         for (size_t g = 0; g < ks->fold_alias.size(); g++)

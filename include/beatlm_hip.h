@@ -325,8 +325,10 @@ uint64_t bl_kernels_packs_made(const bl_kernels *kernels);
 /* Bytes of device memory the kernels hold beside the plan's arenas, in one
  * allocation made by bl_kernels_create (0: none): packed weights, split-k
  * partial sums, attention scratch, the folded LayerNorms' statistics and
- * planes, placed by lifetime as the plan places tensors in an arena (items of
- * disjoint kernel spans share bytes). No counterpart in the reference, whose
+ * planes, and activations moved out of the arenas (a resampling's input that
+ * the plan lays under the product which blends it), placed by lifetime as the
+ * plan places tensors in an arena (items of disjoint kernel spans share bytes,
+ * moved activations with none). No counterpart in the reference, whose
  * kernels hold no memory of their own; with the arenas' one allocation, a
  * program's device memory is these two allocations. */
 uint64_t bl_kernels_workspace_bytes(const bl_kernels *kernels);

@@ -132,3 +132,59 @@ def test_attention_over_a_projection_of_a_resampling(ctx, h, w, oh, ow, heads, m
             ctx.synchronize()
             qkv = oracle.matmul(oracle.resize_bilinear(x, h, w, oh, ow, 64), wq, bq, t, 64, n)
             compare(net.read(105), oracle.attention(qkv, t, heads, 64, 0.125), math, f"{net.labels}, input {seed}")
+
+
+def fused_stage(ctx, math, sets):
+    """conv 256 -> 64, conv 64 -> 64 = x, resampled, 1x1 = y, relu: x moves to
+    the workspace, since the plan lays y over it."""
+    h, w, oh, ow = 8, 8, 16, 16
+    arrays = [stored(math, a) for a in (oracle.fan_in_weights(51, 9 * 256 * 64, 9 * 256), oracle.fan_in_weights(52, 9 * 64 * 64, 9 * 64),
+                                        oracle.fan_in_weights(53, 64 * 64, 64), oracle.uniform(54, 64, -0.1, 0.1))]
+    ops = [(ir.op(ir.OP_CONV3X3, [0, 1, ir.NONE], [h, w, 256, 64, 1]), ir.ACTIVATION),
+           (ir.op(ir.OP_CONV3X3, [100, 2, ir.NONE], [h, w, 64, 64, 1]), ir.ACTIVATION),
+           (ir.op(ir.OP_RESIZE_BILINEAR, [101], [h, w, oh, ow, 64]), ir.ACTIVATION),
+           (ir.op(ir.OP_MATMUL, [102, 3, 4], [oh * ow, 64, 64]), ir.ACTIVATION),
+           (ir.op(ir.OP_RESIZE_BILINEAR, [103], [oh, ow, 5, 7, 64]), ir.OUTPUT)]
+    net = Net(ctx, [(ir.INPUT, h * w * 256)] + [(ir.WEIGHT, a.size) for a in arrays], ops, math, sets)
+    assert net.overlap(101, 103) and "> workspace" in net.labels[1] and "< resize 2" in net.labels[3], net.labels
+    for i, a in enumerate(arrays):
+        net.write(1 + i, a)
+
+    def want(x):
+        y = oracle.conv3x3(x, arrays[0], None, h, w, 256, 64, 1)
+        y = oracle.resize_bilinear(oracle.conv3x3(y, arrays[1], None, h, w, 64, 64, 1), h, w, oh, ow, 64)
+        return oracle.resize_bilinear(oracle.matmul(y, arrays[2], arrays[3], oh * ow, 64, 64), oh, ow, 5, 7, 64)
+
+    return net, want, [stored(math, oracle.uniform(55 + s, h * w * 256, -2.0, 2.0)) for s in range(3)]
+
+
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+def test_a_moved_tensor_follows_each_new_input(ctx, math):
+    net, want, xs = fused_stage(ctx, math, 1)
+    with net:
+        for x in xs:
+            net.write(0, x)
+            net.kernels.encode_all()
+            ctx.synchronize()
+            compare(net.read(104), want(x), math, f"{net.labels}")
+
+
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+def test_a_moved_tensor_outlives_another_sets_kernels(ctx, math):
+    """Every kernel of set 1 between the moved tensor's writer and its reader
+    of set 0 (on the f32 matrix cores the first convolution splits k: its
+    partial sums lie in the workspace too)."""
+    net, want, xs = fused_stage(ctx, math, 2)
+    with net:
+        assert math != "f32" or "splitk" in net.labels[0], net.labels
+        for s in (0, 1):
+            net.write(0, xs[s], s)
+        for k in (0, 1):
+            net.kernels.encode(k, 0)
+        for k in range(5):
+            net.kernels.encode(k, 1)
+        for k in (2, 3, 4):
+            net.kernels.encode(k, 0)
+        ctx.synchronize()
+        for s in (0, 1):
+            compare(net.read(104, s), want(xs[s]), math, f"set {s}, {net.labels}")

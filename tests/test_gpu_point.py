@@ -4,7 +4,7 @@ slice, columns that end inside a 64-wide block, rows that end inside a
 16-pixel tile), the 1x1 convolution that blends its resampled input's corners
 as it loads them, the direct convolution that adds up its channels for a
 one-column product, and the taps' LayerNorm that writes the feature map; each
-run twice, so that a moved tensor's second pass is checked too.
+run twice over the same inputs.
 
 Tolerance for f32 storage: |got - want| <= 1e-4 + 1e-4 |want|
 (reference.rs:22-24); for f16 storage, max abs error <= 2e-2 against the
@@ -69,8 +69,8 @@ def test_a_transposed_convolution_as_a_product_matches_the_oracle(ctx, h, w, cin
                                              (3, 8, 1, 1, 40, 16)])
 @pytest.mark.parametrize("math", MATHS)
 def test_a_resampling_blended_into_its_product_matches_the_oracle(ctx, ih, iw, oh, ow, c, n, math):
-    """conv -> resize -> 1x1 -> relu: the convolution's output is the internal
-    tensor that may move."""
+    """conv -> resize -> 1x1 -> relu, the product writing the program's output
+    (one that lies over the convolution's: test_gpu_plans.py)."""
     arrays = [oracle.uniform(11 + c, ih * iw * c, -2.0, 2.0), oracle.fan_in_weights(12, 9 * c * c, 9 * c), oracle.fan_in_weights(13 + n, c * n, c),
               oracle.uniform(14, n, -0.1, 0.1)]
     ops = [ir.op(ir.OP_CONV3X3, [0, 1, ir.NONE], [ih, iw, c, c, 1]), ir.op(ir.OP_RESIZE_BILINEAR, [H_], [ih, iw, oh, ow, c]),
