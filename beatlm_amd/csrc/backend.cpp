@@ -822,6 +822,12 @@ void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint3
     }
 }
 
+// Whether launch L's output lies apart from the `bytes` at p: a kernel that
+// writes L's output in L's place may then read them throughout.
+bool apart(const Launch &L, const void *p, uint64_t bytes) {
+    return (const char *)p >= L.out_hi || (const char *)p + bytes <= L.out_lo;
+}
+
 // An internal tensor's uses: its one writer and one reader among the kernels
 // (-1: none or several), the reader through binding `read_binding` alone.
 struct OneUse {
@@ -873,12 +879,9 @@ void plan_maps(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
         for (uint32_t si = 0; si < ks->sets && ok; si++) {
             const Launch &L = ks->kernels[li].per_set[si], &Q = ks->kernels[qi].per_set[si];
             const uint64_t esz = L.f16 ? 2 : 4;
-            auto apart = [&](const void *p, uint64_t elements) {
-                return (const char *)p >= Q.out_hi || (const char *)p + elements * esz <= Q.out_lo;
-            };
             ok = L.family == Family::LAYER_NORM && L.fold < 0 && Q.family == Family::ELEMENT && (const void *)Q.el.a == L.ln.y &&
-                 (L.ln.channels * esz) % 16 == 0 && apart(L.ln.x, (uint64_t)L.ln.rows * L.ln.channels) &&
-                 apart(L.ln.gamma, L.ln.channels) && apart(L.ln.beta, L.ln.channels);
+                 (L.ln.channels * esz) % 16 == 0 && apart(Q, L.ln.x, (uint64_t)L.ln.rows * L.ln.channels * esz) &&
+                 apart(Q, L.ln.gamma, L.ln.channels * esz) && apart(Q, L.ln.beta, L.ln.channels * esz);
         }
         if (!ok) continue;
         for (uint32_t si = 0; si < ks->sets; si++) {
@@ -998,7 +1001,7 @@ void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32
 // adds up each pixel's channels in its epilogue and the product launches
 // nothing. Both whole, the channels (one block of the convolution's) an
 // internal tensor that nothing else reads, and the product's output apart from
-// the convolution's image. The channels' round trip through memory goes too: 34
+// all that the convolution reads (its weights are packed). The channels' round trip through memory goes too: 34
 // MB at 518 x 518 in f32, the decoder 385 -> 379 us, in f16 286 -> 279.
 void plan_dots(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t *internal, uint32_t n_internal) {
     if (!n_internal || getenv("BL_NO_DOT_FUSION")) return;
@@ -1015,14 +1018,13 @@ void plan_dots(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
         bool ok = true;
         for (uint32_t si = 0; si < ks->sets && ok; si++) {
             const Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
-            const uint64_t image = (uint64_t)P.gemm.p0 * P.gemm.p1 * P.gemm.p2 * (P.f16 ? 2 : 4);
+            const uint64_t esz = P.f16 ? 2 : 4, image = (uint64_t)P.gemm.p0 * P.gemm.p1 * P.gemm.p2 * esz;
             ok = P.family == Family::GEMM && P.tile == TILE_CONV3 && P.gemm.n == CD_NB && !P.gemm.c_planes && Q.family == Family::GEMV &&
                  Q.gv.n == 1 && Q.gv.k == CD_NB && Q.gv.a == P.gemm.c && Q.gv.row0 == 0 && Q.gv.row1 == P.gemm.m && Q.f16 == P.f16 &&
-                 (Q.out_hi <= (const char *)P.gemm.a || (const char *)P.gemm.a + image <= Q.out_lo);
+                 apart(Q, P.gemm.a, image) && (!P.gemm.bias || apart(Q, P.gemm.bias, P.gemm.n * esz));
             for (int e = 0; e < P.gemm.epi.n && ok; e++)
-                if (P.gemm.epi.kind[e] == BL_EPI_ADD)
-                    ok = Q.out_hi <= (const char *)P.gemm.epi.operand[e] ||
-                         (const char *)P.gemm.epi.operand[e] + (P.out_hi - P.out_lo) <= Q.out_lo;
+                if (const void *o = P.gemm.epi.operand[e])
+                    ok = apart(Q, o, P.gemm.epi.kind[e] == BL_EPI_ADD ? P.out_hi - P.out_lo : P.gemm.epi.channels[e] * esz);
         }
         if (!ok) continue;
         for (uint32_t si = 0; si < ks->sets; si++) {

@@ -188,3 +188,35 @@ def test_a_moved_tensor_outlives_another_sets_kernels(ctx, math):
         ctx.synchronize()
         for s in (0, 1):
             compare(net.read(104, s), want(xs[s]), math, f"set {s}, {net.labels}")
+
+
+@pytest.mark.parametrize("operand", ["bias", "channel scale"])
+@pytest.mark.parametrize("math", ["bf16x3", "f16"], indirect=True)
+def test_a_one_column_product_over_what_its_convolution_reads(ctx, operand, math):
+    """The plan lays the product's output over the convolution's bias (its
+    channel scale): the convolution's workgroups all read those, so the
+    product keeps a launch of its own."""
+    h, w = 130, 255
+    wc, ch, w1, b1 = (stored(math, a) for a in (oracle.fan_in_weights(62, 9 * 32 * 32, 9 * 32), oracle.uniform(63, 32, 0.5, 1.5),
+                                                oracle.fan_in_weights(64, 32, 32), oracle.uniform(65, 1, -0.1, 0.1)))
+    x = stored(math, oracle.uniform(61, h * w * 32, -2.0, 2.0))
+    ops = [(ir.op(ir.OP_RELU, [2], [32]), ir.ACTIVATION)]
+    if operand == "bias":
+        ops += [(ir.op(ir.OP_CONV3X3, [0, 1, 100], [h, w, 32, 32, 1]), ir.ACTIVATION)]
+    else:
+        ops += [(ir.op(ir.OP_CONV3X3, [0, 1, ir.NONE], [h, w, 32, 32, 1]), ir.ACTIVATION),
+                (ir.op(ir.OP_CHANNEL_SCALE, [101, 100], [h * w, 32]), ir.ACTIVATION)]
+    c = 100 + len(ops) - 1
+    ops += [(ir.op(ir.OP_MATMUL, [c, 3, 4], [h * w, 32, 1]), ir.ACTIVATION), (ir.op(ir.OP_RESIZE_BILINEAR, [c + 1], [h, w, 20, 30, 1]), ir.OUTPUT)]
+    with Net(ctx, [(ir.INPUT, x.size), (ir.WEIGHT, wc.size), (ir.WEIGHT, 32), (ir.WEIGHT, 32), (ir.WEIGHT, 1)], ops, math) as net:
+        assert net.overlap(100, c + 1) and "direct" in net.labels[1], net.labels
+        assert "product" not in net.labels[1], net.labels
+        for i, a in enumerate((x, wc, ch, w1, b1)):
+            net.write(i, a)
+        net.kernels.encode_all()
+        ctx.synchronize()
+        y = oracle.conv3x3(x, wc, ch if operand == "bias" else None, h, w, 32, 32, 1)
+        if operand != "bias":
+            y = oracle.channel_scale(y, ch)
+        want = oracle.resize_bilinear(oracle.matmul(y, w1, b1, h * w, 32, 1), h, w, 20, 30, 1)
+        compare(net.read(c + 2), want, math, f"{net.labels}")
