@@ -579,6 +579,14 @@ bool shape_of(const bl_spec &s, Shape &sh, std::string &why) {
     }
 }
 
+// Whether a spec covers all of its output: one part, which a caller may also
+// give less than the split dimension.
+bool whole(const bl_spec &s) {
+    Shape sh;
+    std::string why;
+    return s.part.count == 1 && s.part.start == 0 && shape_of(s, sh, why) && s.part.end == sh.extent;
+}
+
 uint64_t round4(uint64_t bytes) { return (bytes + 3) / 4 * 4; }
 
 }  // namespace
@@ -867,8 +875,8 @@ void plan_maps(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
     for (uint32_t qi = 1; qi < n; qi++) {
         const uint32_t li = qi - 1;
         const bl_spec &qs = specs[qi], &ls = specs[li];
-        if (qs.main != BL_MAIN_TOKENS_TO_MAP || qs.part.count != 1 || qs.n_epilogue || ls.main != BL_MAIN_LAYER_NORM ||
-            ls.part.count != 1 || ls.n_epilogue)
+        if (qs.main != BL_MAIN_TOKENS_TO_MAP || !whole(qs) || qs.n_epilogue || ls.main != BL_MAIN_LAYER_NORM || !whole(ls) ||
+            ls.n_epilogue)
             continue;
         const uint32_t t = ls.bindings[ls.n_bindings - 1].tensor;
         const OneUse u = one_use(specs, n, t);
@@ -920,7 +928,7 @@ void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32
     for (uint32_t pi = 1; pi < n; pi++) {
         const uint32_t qi = pi - 1;
         const bl_spec &ps = specs[pi], &qs = specs[qi];
-        if (ps.main != BL_MAIN_MATMUL || ps.part.count != 1 || qs.main != BL_MAIN_RESIZE_BILINEAR || qs.part.count != 1 || qs.n_epilogue)
+        if (ps.main != BL_MAIN_MATMUL || !whole(ps) || qs.main != BL_MAIN_RESIZE_BILINEAR || !whole(qs) || qs.n_epilogue)
             continue;
         const uint32_t t = qs.bindings[qs.n_bindings - 1].tensor, xt = qs.bindings[qs.reads[0]].tensor;
         const OneUse u = one_use(specs, n, t), ux = one_use(specs, n, xt);
@@ -960,7 +968,7 @@ void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32
             if (P.out_lo < (const char *)pa.x + x_bytes && (const char *)pa.x < P.out_hi) move = true;
         }
         if (ok && move) {
-            ok = is_internal(xt) && ux.reader == (int)qi && ux.writer >= 0 && ux.writer < (int)qi && specs[ux.writer].part.count == 1;
+            ok = is_internal(xt) && ux.reader == (int)qi && ux.writer >= 0 && ux.writer < (int)qi && whole(specs[ux.writer]);
             for (uint32_t si = 0; si < ks->sets && ok; si++) {
                 const Launch &W = ks->kernels[ux.writer].per_set[si];
                 ok = W.family == Family::GEMM && !W.point && W.fold < 0 && !W.gemm.cls_out && !W.gemm.flash_ops && W.gemm.c == args[si].x;
@@ -1010,7 +1018,7 @@ void plan_dots(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
     for (uint32_t qi = 1; qi < n; qi++) {
         const uint32_t pi = qi - 1;
         const bl_spec &qs = specs[qi], &ps = specs[pi];
-        if (qs.main != BL_MAIN_MATMUL || qs.part.count != 1 || ps.main != BL_MAIN_CONV3X3 || ps.part.count != 1) continue;
+        if (qs.main != BL_MAIN_MATMUL || !whole(qs) || ps.main != BL_MAIN_CONV3X3 || !whole(ps)) continue;
         const uint32_t t = ps.bindings[ps.n_bindings - 1].tensor;
         const OneUse u = one_use(specs, n, t);
         if (!std::binary_search(ids.begin(), ids.end(), t) || u.writer != (int)pi || u.reader != (int)qi || u.read_binding != qs.reads[0])
@@ -1868,7 +1876,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                 L.dp.end = (uint64_t)pt.end * sh.per_unit;
                 L.dp.epi = epi;
                 variant = "per-element";
-                if (ct && pt.count == 1 && !getenv("BL_NO_POINT")) {
+                if (ct && whole(s) && !getenv("BL_NO_POINT")) {
                     // A whole transposed convolution of few channels: a product
                     // over the input pixels (k_point.hip), in f32 on the matrix
                     // cores for f32 storage as the vector ALUs had it (us over 37 x

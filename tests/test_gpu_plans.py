@@ -220,3 +220,56 @@ def test_a_one_column_product_over_what_its_convolution_reads(ctx, operand, math
             y = oracle.channel_scale(y, ch)
         want = oracle.resize_bilinear(oracle.matmul(y, w1, b1, h * w, 32, 1), h, w, 20, 30, 1)
         compare(net.read(c + 2), want, math, f"{net.labels}")
+
+
+def part(specs, k, start, end):
+    specs[k].part = hip.Part(0, 1, start, end)
+
+
+@pytest.mark.parametrize("which", ["map", "layernorm", "resampled product", "resampling", "one column", "transposed"])
+@pytest.mark.parametrize("math", ["bf16x3", "f16"], indirect=True)
+def test_a_lone_part_that_does_not_cover_its_tensor_writes_its_own_range(ctx, which, math):
+    """Part 1 of 1 may cover less than its tensor: the rest of the output stays
+    as the host left it (outputs here start at 7)."""
+    u = lambda seed, n: stored(math, oracle.uniform(seed, n, -1.0, 1.0))
+    if which in ("map", "layernorm"):
+        t, d = 26, 64
+        arrays = [u(71, t * d), u(72, d), u(73, d)]
+        ops = [(ir.op(ir.OP_LAYER_NORM, [0, 1, 2], [t, d], EPS), ir.ACTIVATION), (ir.op(ir.OP_TOKENS_TO_MAP, [100], [5, 5, d]), ir.OUTPUT)]
+        full = oracle.layernorm(*arrays, t, d, EPS).reshape(t, d)[1:].reshape(-1)
+        if which == "map":
+            change, lo, hi = (lambda s: part(s, 1, 3 * d, 17 * d)), 3 * d, 17 * d
+        else:
+            # Rows 1 .. 9 alone are the LayerNorm's: map rows 0 .. 8 are checked.
+            change, lo, hi = (lambda s: part(s, 0, 0, 10)), 0, 9 * d
+    elif which in ("resampled product", "resampling"):
+        arrays = [u(74, 64 * 64), u(75, 64 * 64), u(76, 64)]
+        ops = [(ir.op(ir.OP_RESIZE_BILINEAR, [0], [8, 8, 16, 16, 64]), ir.ACTIVATION), (ir.op(ir.OP_MATMUL, [100, 1, 2], [256, 64, 64]), ir.OUTPUT)]
+        full = oracle.matmul(oracle.resize_bilinear(arrays[0], 8, 8, 16, 16, 64), arrays[1], arrays[2], 256, 64, 64)
+        if which == "resampled product":
+            change, lo, hi = (lambda s: part(s, 1, 64, 128)), 64 * 64, 128 * 64
+        else:
+            change, lo, hi = (lambda s: part(s, 0, 0, 100)), 0, 100 * 64
+    elif which == "one column":
+        h, w = 130, 255
+        arrays = [u(77, h * w * 32), stored(math, oracle.fan_in_weights(78, 9 * 32 * 32, 9 * 32)), u(79, 32), u(80, 1)]
+        ops = [(ir.op(ir.OP_CONV3X3, [0, 1, ir.NONE], [h, w, 32, 32, 1]), ir.ACTIVATION), (ir.op(ir.OP_MATMUL, [100, 2, 3], [h * w, 32, 1]), ir.OUTPUT)]
+        full = oracle.matmul(oracle.conv3x3(arrays[0], arrays[1], None, h, w, 32, 32, 1), arrays[2], arrays[3], h * w, 32, 1)
+        change, lo, hi = (lambda s: part(s, 0, 0, 33088)), 0, 33088
+    else:
+        arrays = [u(81, 9 * 9 * 48), u(82, 4 * 48 * 48), u(83, 48)]
+        ops = [(ir.op(ir.OP_CONV_TRANSPOSE, [0, 1, 2], [9, 9, 48, 48, 2]), ir.OUTPUT)]
+        full = oracle.conv_transpose(arrays[0], arrays[1], arrays[2], 9, 9, 48, 48, 2)
+        change, lo, hi = (lambda s: part(s, 0, 50, 201)), 50 * 48, 201 * 48
+    whole = which in ("layernorm", "resampling", "one column")  # the last kernel writes all: the rest of its input is arbitrary
+    out = 100 + len(ops) - 1
+    with Net(ctx, [(ir.INPUT, arrays[0].size)] + [(ir.WEIGHT, a.size) for a in arrays[1:]], ops, math, change=change) as net:
+        for i, a in enumerate(arrays):
+            net.write(i, a)
+        net.write(out, np.full(full.size, 7.0))
+        net.kernels.encode_all()
+        ctx.synchronize()
+        got = net.read(out)
+        compare(got[lo:hi], full[lo:hi], math, f"{net.labels}")
+        assert whole or (np.all(got[:lo] == 7.0) and np.all(got[hi:] == 7.0)), net.labels
+        assert not any("fused" in lab for lab in net.labels), net.labels
