@@ -2038,11 +2038,12 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
             pk.vec_offset = pack_total;
             pack_total += align256(fold_vec_bytes(pk.n_pad));
         }
-        // Written by a kernel of this program: packed again before every launch.
-        for (uint32_t ki = 0; ki < n && !pk.dynamic; ki++) {
-            const bl_binding &o = specs[ki].bindings[specs[ki].n_bindings - 1];
-            if (pk.reads(o.arena, o.offset, o.size)) pk.dynamic = true;
-        }
+        // Written by a kernel of this program, in any set: packed again before every launch.
+        for (uint32_t ki = 0; ki < n && !pk.dynamic; ki++)
+            for (uint32_t si = 0; si < n_sets && !pk.dynamic; si++) {
+                const bl_binding o = resolve(specs[ki], specs[ki].n_bindings - 1, sets[si]);
+                pk.dynamic = pk.reads(o.arena, o.offset, o.size);
+            }
     }
     for (const Pack &pk : ks->packs)
         if (pk.used && pk.dynamic) ks->graphs_ok = false;

@@ -273,3 +273,26 @@ def test_a_lone_part_that_does_not_cover_its_tensor_writes_its_own_range(ctx, wh
         compare(got[lo:hi], full[lo:hi], math, f"{net.labels}")
         assert whole or (np.all(got[:lo] == 7.0) and np.all(got[hi:] == 7.0)), net.labels
         assert not any("fused" in lab for lab in net.labels), net.labels
+
+
+@pytest.mark.parametrize("product", ["transposed convolution", "matmul"])
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+def test_weights_that_a_kernel_writes_are_packed_again_in_every_set(ctx, product, math):
+    """The weights are a kernel's output, at a place of its own in each set."""
+    if product == "matmul":
+        x, n = stored(math, oracle.uniform(91, 40 * 64, -1.0, 1.0)), 64 * 64
+        o = ir.op(ir.OP_MATMUL, [0, 100, ir.NONE], [40, 64, 64])
+        want = lambda w: oracle.matmul(x, w, None, 40, 64, 64)
+    else:
+        x, n = stored(math, oracle.uniform(92, 9 * 9 * 48, -1.0, 1.0)), 4 * 48 * 48
+        o = ir.op(ir.OP_CONV_TRANSPOSE, [0, 100, ir.NONE], [9, 9, 48, 48, 2])
+        want = lambda w: oracle.conv_transpose(x, w, None, 9, 9, 48, 48, 2)
+    with Net(ctx, [(ir.INPUT, x.size), (ir.INPUT, n)], [(ir.op(ir.OP_RELU, [1], [n]), ir.ACTIVATION), (o, ir.OUTPUT)], math, 2) as net:
+        for seed in (93, 94):
+            for s in (0, 1):
+                w = stored(math, oracle.uniform(seed + 10 * s, n, -0.2, 0.2))
+                net.write(0, x, s)
+                net.write(1, w, s)
+                net.kernels.encode_all(s)
+                ctx.synchronize()
+                compare(net.read(101, s), want(np.maximum(w, 0)), math, f"set {s}, weights {seed}: {net.labels}")
