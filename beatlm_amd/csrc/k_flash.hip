@@ -1065,6 +1065,9 @@ __global__ __launch_bounds__(SMALL_THREADS) void attn_small_kernel(FlashArgs a) 
     }
 
     const uint64_t plane = (uint64_t)H * tpad * HD;
+    // The f32 values come through a buffer of qkv's bytes: those past the last key read as zeros, as the other
+    // maths' operands hold (a zero probability times an infinity is no zero).
+    const auto values = __builtin_amdgcn_make_buffer_rsrc((void *)qkv, 0, Tn * row_stride * 4, 0x00027000);
     auto load = [&](uint32_t grp, SmallKv<M> &kv) {
         const uint32_t key0 = SKEYS * grp;
         if constexpr (M == Math::F32) {
@@ -1077,10 +1080,10 @@ __global__ __launch_bounds__(SMALL_THREADS) void attn_small_kernel(FlashArgs a) 
                 for (int i = 0; i < 4; i++) kv.k[kb][i] = *(const f32x4 *)(kp + 4 * i);
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const uint32_t vkey = min(key0 + 16 * kb + 4 * g + r, Tn - 1);
-                    const float *vp = (const float *)qkv + (uint64_t)vkey * row_stride + (2 * H + head) * HD + l16;
+                    const uint32_t at = 4 * ((key0 + 16 * kb + 4 * g + r) * row_stride + (2 * H + head) * HD + l16);
 #pragma unroll
-                    for (int db = 0; db < 4; db++) kv.v[kb][r][db] = vp[16 * db];
+                    for (int db = 0; db < 4; db++)
+                        kv.v[kb][r][db] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(values, at + 64 * db, 0, 0));
                 }
             }
         } else {
@@ -1104,7 +1107,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void attn_small_kernel(FlashArgs a) 
     float m[QB], l[QB];
 #pragma unroll
     for (int b = 0; b < QB; b++) {
-        m[b] = -INFINITY;
+        m[b] = -__FLT_MAX__;  // finite: keys that score -inf have probability zero, whichever come first
         l[b] = 0.0f;
 #pragma unroll
         for (int db = 0; db < 4; db++) o[b][db] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1165,7 +1168,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void attn_small_kernel(FlashArgs a) 
                     mx = fmaxf(mx, s[kb][r]);
                 }
             mx = max_xor32(fmaxf(mx, __shfl_xor(mx, 16, WAVE)));
-            const float m_new = fmaxf(m[b], mx);  // finite: every group holds a key < T
+            const float m_new = fmaxf(m[b], mx);
             const float alpha = __builtin_amdgcn_exp2f(m[b] - m_new);
             m[b] = m_new;
             float p[8], sum = 0.0f;
@@ -1230,7 +1233,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void attn_small_kernel(FlashArgs a) 
     // Four columns of one query an invocation, the waves in order.
     if (tid >= QROWS * (HD / 4)) return;
     const uint32_t r = tid / (HD / 4), d = tid % (HD / 4) * 4, q = q0 + r;
-    float mt = -INFINITY;
+    float mt = -__FLT_MAX__;
 #pragma unroll
     for (int w = 0; w < SW; w++) mt = fmaxf(mt, sml[w][r][0]);
     float lt = 0.0f;
@@ -1331,6 +1334,8 @@ hipError_t launch_flash(const FlashArgs &a, Math m, hipStream_t s) {
 // 25.7 / 15.5; 12 heads, 626: 15.7 / 23.4 / 14.3). BL_FLASH_SMALL: 0, 1 or 2
 // blocks whatever the size.
 static uint32_t small_blocks(Math m, uint32_t tokens, uint32_t heads, uint32_t rows, uint32_t compute_units) {
+    // The f32 kernel's byte offsets into qkv are 32-bit, up to a group past its end.
+    if (m == Math::F32 && (uint64_t)(tokens + SKEYS) * heads * 3 * HD * 4 >= (1ull << 32)) return 0;
     if (const char *knob = getenv("BL_FLASH_SMALL")) return std::min(2, std::max(0, atoi(knob)));
     if (getenv("BL_FLASH_MERGE_LAUNCH") || (m == Math::SPLIT && tokens > 640)) return 0;
     for (uint32_t b = 1; b <= 2; b++)

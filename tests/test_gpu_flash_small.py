@@ -2,7 +2,9 @@
 32 queries, its waves splitting the keys in groups of 32) against the oracle:
 one token, tokens that end inside a query block, a key group and a round of
 eight groups, exactly on them, and three rounds; a kernel of several parts;
-and a block whose attention reads the operands its QKV projection wrote.
+and a block whose attention reads the operands its QKV projection wrote; and
+infinities, in scores and values (not in bf16x3, where an infinity has no hi
+and lo parts).
 
 Tolerance for f32 storage: |got - want| <= 1e-4 + 1e-4 |want|
 (reference.rs:22-24); for f16 storage, max abs error <= 2e-2 against the
@@ -90,3 +92,57 @@ def test_a_small_blocks_attention_reads_its_projections_operands(ctx, t, math):
     if math == "f16":
         x, w = (x.astype(np.float16).astype(np.float32), {k: v.astype(np.float16).astype(np.float32) for k, v in w.items()})
     compare(got, oracle.vit_block(x, w, t, h, d // h, mlp, 1e-6), math, f"block of {t} tokens")
+
+
+@pytest.mark.parametrize("t,first,count", [(70, 32, 32), (290, 0, 64), (300, 128, 100)])
+@pytest.mark.parametrize("math", ["f32", "f16"], indirect=True)
+@pytest.mark.parametrize("blocks", ["1", "2"])
+def test_keys_with_scores_of_minus_infinity_take_no_part(ctx, monkeypatch, t, first, count, math, blocks):
+    """Keys first .. first + count - 1 score -inf against every query (whole
+    groups of 32 of them): their probabilities are zero, as a softmax over
+    the row has them."""
+    monkeypatch.setenv("BL_FLASH_SMALL", blocks)
+    qkv = oracle.uniform(t, t * 192, -3.0, 3.0)
+    if math == "f16":
+        qkv = qkv.astype(np.float16)
+    v = qkv.reshape(t, 3, 64)
+    v[:, 0, 5] = 1.0
+    v[first : first + count, 1, 5] = -np.inf
+    kept = np.delete(v, np.s_[first : first + count], 0)
+    s = v[:, 0].astype(np.float64) @ kept[:, 1].astype(np.float64).T * 0.125
+    p = np.exp(s - s.max(1, keepdims=True))
+    want = (p / p.sum(1, keepdims=True)) @ kept[:, 2].astype(np.float64)
+    prep = ir.prepare(ctx, attention_graph(t, 1, 64), dtype=hip.F16 if math == "f16" else hip.F32)
+    try:
+        assert "keys over waves" in prep.kernels.label(0)
+        prep.write(X, qkv)
+        prep.run()
+        ctx.synchronize()
+        compare(prep.read(Y).astype(np.float32), want.reshape(-1).astype(np.float32), math, f"t={t}")
+    finally:
+        prep.close()
+
+
+@pytest.mark.parametrize("t", [33, 257, 290])
+@pytest.mark.parametrize("math", ["f32", "f16"], indirect=True)
+@pytest.mark.parametrize("blocks", ["1", "2"])
+def test_an_infinite_value_of_the_last_token_stays_infinite(ctx, monkeypatch, t, math, blocks):
+    """One column of the last token's value is +inf: that column of every
+    query's output is, and no other column is touched."""
+    monkeypatch.setenv("BL_FLASH_SMALL", blocks)
+    qkv = oracle.uniform(t + 1, t * 192, -1.0, 1.0)
+    if math == "f16":
+        qkv = qkv.astype(np.float16)
+    qkv.reshape(t, 3, 64)[-1, 2, 9] = np.inf
+    want = oracle.attention(np.where(np.isinf(qkv), 0, qkv).astype(np.float32), t, 1, 64, 0.125).reshape(t, 64)
+    prep = ir.prepare(ctx, attention_graph(t, 1, 64), dtype=hip.F16 if math == "f16" else hip.F32)
+    try:
+        prep.write(X, qkv)
+        prep.run()
+        ctx.synchronize()
+        got = prep.read(Y).astype(np.float32).reshape(t, 64)
+        assert np.all(np.isposinf(got[:, 9])), got[:4, 9]
+        rest = np.arange(64) != 9
+        compare(got[:, rest].reshape(-1), want[:, rest].reshape(-1), math, f"t={t}")
+    finally:
+        prep.close()
