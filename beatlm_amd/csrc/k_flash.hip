@@ -1323,24 +1323,52 @@ hipError_t launch_flash(const FlashArgs &a, Math m, hipStream_t s) {
     }
 }
 
-// 16-query blocks per workgroup of attn_small_kernel, 0 for the other kernels:
-// the fewest (1 or 2) whose workgroups all run at once, one per CU; a second
-// round doubles its time. It beats the 256-query tiles over all such sizes in
-// f16 (us, 256-query tiles / 1 block / 2 blocks; 6 heads: 257 tokens 11.4 /
-// 5.0 / 6.0, 626 12.9 / 7.2 / 8.4, 1200 16.0 / 21.2 / 13.2; 16 heads, 500: 15.2
-// / 10.8 / 7.2) and on the f32 matrix cores (257: 17.2 / 9.3 / 14.3; 1025: 38.7
-// / 37.8 / 30.4); in bf16x3, whose keys and values are twice the bytes, up to
-// 640 tokens (6 heads: 257 12.6 / 7.7 / 9.4, 626 14.2 / 12.3 / 14.0, 700 15.1 /
-// 25.7 / 15.5; 12 heads, 626: 15.7 / 23.4 / 14.3). BL_FLASH_SMALL: 0, 1 or 2
-// blocks whatever the size.
-static uint32_t small_blocks(Math m, uint32_t tokens, uint32_t heads, uint32_t rows, uint32_t compute_units) {
+// 16-query blocks per workgroup of attn_small_kernel, 0 for the other kernels
+// (planned in p): the fewest (1 or 2) whose workgroups all run at once, one
+// per CU (a second round doubles its time), if that is the faster kernel. Its
+// time grows with the tokens alone, however few the rows (a part's), the
+// others' with the tiles each CU walks, so both are estimated (us, on what was
+// measured of 257 to 8192 tokens, 1 to 16 heads, whole and in 2 to 4 parts;
+// the two are within 9% of each other where the estimate errs):
+//   1 block: f16 3.2 + 7.1 per 1000 tokens, f32 matrix cores 5.0 + 13
+//   2 blocks: f16 4.0 + 7.5, f32 matrix cores 4.5 + 20
+//   256-query tiles, f16: 12.5 + 1.6 per key tile of a run
+//   f32 matrix cores: 17 + 3.2 per key tile of a split while the workgroups
+//   run one to a CU, else 14 + 2.65 times their rounds per key tile.
+// us a part, others / 1 block / 2 blocks (of a whole kernel: 1 part):
+//   f16, 6 heads: 257 tokens 11.5 / 5.2 / 6.1; 1200 16.4 / 22.2 / 14.0;
+//     1370 in 2 parts 15.1 / 24.0 / 14.0, in 4 13.6 / 12.6 / 13.6; 2501 in 2
+//     parts 21.1 / 40.7 / 23.5, in 4 17.5 / 21.4 / 22.3; 5477 in 4 parts 32.2 /
+//     82.7 / 45.6; 16 heads, 1370 in 3 17.3 / 24.5 / 14.6; 1 head, 8192 38.0 /
+//     119.7 / 64.9
+//   f32 matrix cores, 6 heads: 257 17.7 / 8.4 / 12.7; 1370 in 2 38.9 / 41.8 /
+//     32.8; 2501 in 3 58.8 / 71.5 / 55.3; 5477 in 4 142 / 146 / 114; 1 head,
+//     8192 in 4 60.8 / 101 / 156
+// In bf16x3, whose keys and values are twice the bytes, it leads up to 640
+// tokens, and up to 448 where the rows are at most 192 (6 heads: 257 12.8 / 8.0
+// / 9.6; 626 14.5 / 12.8 / 14.4, in 4 parts 10.8 / 12.2 / 13.7; 700 15.3 / 26.3 /
+// 15.9; 500 in 3 10.0 / 10.4 / 11.8; 362 in 4 9.0 / 8.9 / 10.4).
+// BL_FLASH_SMALL: 0, 1 or 2 blocks whatever the size.
+static uint32_t small_blocks(const FlashPlan &p, Math m, uint32_t tokens, uint32_t heads, uint32_t rows, uint32_t compute_units) {
     // The f32 kernel's byte offsets into qkv are 32-bit, up to a group past its end.
     if (m == Math::F32 && (uint64_t)(tokens + SKEYS) * heads * 3 * HD * 4 >= (1ull << 32)) return 0;
     if (const char *knob = getenv("BL_FLASH_SMALL")) return std::min(2, std::max(0, atoi(knob)));
-    if (getenv("BL_FLASH_MERGE_LAUNCH") || (m == Math::SPLIT && tokens > 640)) return 0;
-    for (uint32_t b = 1; b <= 2; b++)
-        if ((uint64_t)heads * ((rows + 16 * b - 1) / (16 * b)) <= compute_units) return b;
-    return 0;
+    if (getenv("BL_FLASH_MERGE_LAUNCH")) return 0;
+    uint32_t b = 1;
+    while (b <= 2 && (uint64_t)heads * ((rows + 16 * b - 1) / (16 * b)) > compute_units) b++;
+    if (b > 2) return 0;
+    if (m == Math::SPLIT) return tokens <= (rows > 192 ? 640u : 448u) ? b : 0;
+    const double t = tokens * 1e-3;
+    double small, others;
+    if (m == Math::F16) {
+        small = b == 1 ? 3.2 + 7.1 * t : 4.0 + 7.5 * t;
+        others = 12.5 + 1.6 * (double)p.units / compute_units;
+    } else {
+        const uint64_t wgs = (uint64_t)((rows + 63) / 64) * heads * p.splits, rounds = (wgs + compute_units - 1) / compute_units;
+        small = b == 1 ? 5.0 + 13.0 * t : 4.5 + 20.0 * t;
+        others = (rounds <= 1 ? 17.0 : 14.0) + (double)((tokens + KT - 1) / KT) / p.splits * (rounds <= 1 ? 3.2 : 2.65 * rounds);
+    }
+    return small <= others ? b : 0;
 }
 
 FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uint32_t row1, uint32_t compute_units) {
@@ -1349,7 +1377,6 @@ FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uin
     const uint32_t t_pad = (tokens + KT - 1) / KT * KT;
     const uint32_t kt = t_pad / KT;
     uint64_t extra = 0;
-    p.small = small_blocks(m, tokens, heads, rows, compute_units);
     if (m == Math::F32) {
         const uint32_t wgs = (rows + 63) / 64 * heads;
         // Enough workgroups for two per CU, each split keeping two key tiles or more.
@@ -1390,6 +1417,7 @@ FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uin
         p.counter_bytes = (uint64_t)p.counters * COUNTER_STRIDE * sizeof(uint32_t);
     }
     p.scratch_bytes = operand_bytes(m, heads, t_pad) + extra;
+    p.small = small_blocks(p, m, tokens, heads, rows, compute_units);
     return p;
 }
 

@@ -146,3 +146,27 @@ def test_an_infinite_value_of_the_last_token_stays_infinite(ctx, monkeypatch, t,
         compare(got[:, rest].reshape(-1), want[:, rest].reshape(-1), math, f"t={t}")
     finally:
         prep.close()
+
+
+@pytest.mark.parametrize("math,t,h,parts,few", [
+    ("f16", 1200, 6, 1, True), ("f16", 1370, 6, 4, True), ("f16", 2501, 6, 4, False), ("f16", 5477, 6, 4, False), ("f16", 8192, 1, 1, False),
+    ("f32", 1370, 6, 4, True), ("f32", 5477, 6, 2, False), ("f32", 8192, 1, 4, False),
+    ("bf16x3", 626, 6, 1, True), ("bf16x3", 626, 6, 4, False), ("bf16x3", 362, 6, 4, True), ("bf16x3", 700, 6, 1, False)], indirect=["math"])
+def test_parts_of_a_long_sequence_keep_the_kernel_that_shares_out_its_keys(ctx, math, t, h, parts, few):
+    """The few-token kernel's time grows with the tokens however few a part's
+    rows: every part of one kernel is planned by both (a projection before it,
+    so that the choice is the planner's in f16 and bf16x3 too)."""
+    d, g = 64 * h, ir.Graph()
+    for tid, n in ((0, t * d), (1, 3 * d * d), (2, 3 * d)):
+        g.tensor(tid, ir.WEIGHT if tid else ir.INPUT, n)
+    ops = [ir.op(ir.OP_MATMUL, [0, 1, 2], [t, d, 3 * d]), ir.op(ir.OP_ATTENTION_SCORES, [10], [t, h, 64]),
+           ir.op(ir.OP_SCALE, [11], [t * h * t], 0.125), ir.op(ir.OP_SOFTMAX, [12], [t * h, t]), ir.op(ir.OP_ATTENTION_VALUES, [13, 10], [t, h, 64])]
+    for i, o in enumerate(ops):
+        g.tensor(10 + i, ir.OUTPUT if i == 4 else ir.ACTIVATION, ir.output_elements(o))
+        g.push(o, 10 + i)
+    prep = ir.realise(ctx, g.lower().fuse_attention().split([1, parts]), hip.F16 if math == "f16" else hip.F32)
+    try:
+        labels = [prep.kernels.label(k) for k in range(1, len(prep.kernels))]
+        assert all(("keys over waves" in lab) == few for lab in labels), labels
+    finally:
+        prep.close()
