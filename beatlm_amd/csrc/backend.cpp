@@ -353,6 +353,7 @@ struct Launch {
     // A short product (k_point.hip) in place of the family's own kernel.
     bool point = false;
     PointArgs pt;
+    DotArgs dot{};
     // The output's bytes (what the launch writes, the scratch aside).
     const char *out_lo = nullptr, *out_hi = nullptr;
     // A flash kernel whose QKV projections write its K and Vt (fl.prepped):
@@ -819,7 +820,7 @@ void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint3
             g.epi_mode = 3;
             g.cls_token = Q.el.a;
             g.cls_out = Q.el.y;
-            g.side_epi = Q.el.epi;
+            g.cls_epi = Q.el.epi;
             P.out_lo = Q.out_lo;
             P.out_hi = Q.out_hi;
             Q.fused = true;
@@ -1037,10 +1038,7 @@ void plan_dots(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t 
         if (!ok) continue;
         for (uint32_t si = 0; si < ks->sets; si++) {
             Launch &P = ks->kernels[pi].per_set[si], &Q = ks->kernels[qi].per_set[si];
-            P.gemm.dot_w = Q.gv.b;
-            P.gemm.dot_bias = Q.gv.bias;
-            P.gemm.dot_out = Q.gv.c;
-            P.gemm.side_epi = Q.gv.epi;
+            P.dot = DotArgs{Q.gv.b, Q.gv.bias, Q.gv.c, Q.gv.epi};
             P.out_lo = Q.out_lo;
             P.out_hi = Q.out_hi;
             Q.fused = true;
@@ -2308,7 +2306,7 @@ static hipError_t launch(const Launch &L, hipStream_t s) {
     switch (L.family) {
     case Family::LAYER_NORM: return L.fold_role == FOLD_LAYER_NORM ? hipSuccess : launch_layernorm(L.ln, L.f16, s);
     case Family::GEMM: {
-        const hipError_t e = launch_gemm(L.gemm, L.math, L.tile, s);
+        const hipError_t e = launch_gemm(L.gemm, L.dot, L.math, L.tile, s);
         return e == hipSuccess && L.gemm.ksplit > 1 ? launch_gemm_reduce(L.gemm, L.f16, s) : e;
     }
     case Family::GATHER: return launch_gather(L.ga, L.gather, L.f16, s);

@@ -109,22 +109,25 @@ struct GemmArgs {
     // the plain kernel): c is x's second row, so that the product's rows are
     // x's rows 1 .. m, and the epilogue's added tensors are read one row on
     // likewise; the workgroups of the first row band also write x's first
-    // row, side_epi applied to cls_token [n], at cls_out (x itself), with its
+    // row, cls_epi applied to cls_token [n], at cls_out (x itself), with its
     // block statistics at cls_ln_out and its planes at cls_shadow when the
     // product is a fold's producer. Null cls_out: none.
     const void *cls_token;
     void *cls_out;
     float *cls_ln_out;
     void *cls_shadow;
-    // A product with one output column fused into the direct 3x3 convolution
-    // whose CD_NB channels it reads (the depth head's last 1x1 convolution): a
-    // pixel's channels, through the epilogue and rounded to storage, times
-    // dot_w plus dot_bias (may be null), then side_epi, at dot_out [m]; c is not
-    // written. Null dot_out: none.
-    const void *dot_w, *dot_bias;
-    void *dot_out;
-    // Of the fused prepend or the fused one-column product (never both).
-    EpilogueArgs side_epi;
+    EpilogueArgs cls_epi;
+};
+
+// A product with one output column fused into the direct 3x3 convolution
+// whose CD_NB channels it reads (the depth head's last 1x1 convolution): a
+// pixel's channels, through the convolution's epilogue and rounded to storage,
+// times w plus bias (may be null), then epi, at out [m]; the convolution's c is
+// not written. Null out: none.
+struct DotArgs {
+    const void *w, *bias;
+    void *out;
+    EpilogueArgs epi;
 };
 
 hipError_t launch_gemm_reduce(const GemmArgs &a, bool f16, hipStream_t s);
@@ -320,13 +323,18 @@ hipError_t launch_gemv(const GemvArgs &a, bool f16, hipStream_t s);
 hipError_t launch_gemm_f32(const GemmArgs &a, int tile, hipStream_t s);
 hipError_t launch_gemm_split(const GemmArgs &a, int tile, hipStream_t s);
 hipError_t launch_gemm_f16(const GemmArgs &a, int tile, hipStream_t s);
+hipError_t launch_conv_split(const GemmArgs &a, const DotArgs &dot, hipStream_t s);
+hipError_t launch_conv_f16(const GemmArgs &a, const DotArgs &dot, hipStream_t s);
 hipError_t launch_pack_f32(const PackArgs &a, hipStream_t s);
 hipError_t launch_pack_split(const PackArgs &a, hipStream_t s);
 hipError_t launch_pack_f16(const PackArgs &a, hipStream_t s);
 hipError_t launch_gemm_wave(const GemmArgs &a, Math m, int tile, hipStream_t s);
 inline bool gemm_tile_wave(int t);
-inline hipError_t launch_gemm(const GemmArgs &a, Math m, int tile, hipStream_t s) {
+inline bool gemm_tile_direct(int t);
+inline hipError_t launch_gemm(const GemmArgs &a, const DotArgs &dot, Math m, int tile, hipStream_t s) {
     if (a.row1 <= a.row0) return hipSuccess;
+    if (gemm_tile_direct(tile))
+        return m == Math::F32 ? hipErrorInvalidValue : m == Math::SPLIT ? launch_conv_split(a, dot, s) : launch_conv_f16(a, dot, s);
     if (gemm_tile_wave(tile)) return launch_gemm_wave(a, m, tile, s);
     return m == Math::F32 ? launch_gemm_f32(a, tile, s)
          : m == Math::SPLIT ? launch_gemm_split(a, tile, s) : launch_gemm_f16(a, tile, s);
@@ -412,6 +420,7 @@ __host__ inline bool gemm_wave_fits(const GemmArgs &a, Math m) {
 enum GemmTile : int { TILE_64x64 = 0, TILE_32x64 = 1, TILE_64x128 = 2, TILE_128x64 = 3, TILE_128x32 = 4, TILE_64x96 = 5, TILE_CONV3 = 6, TILE_W16x32 = 7, TILE_W32x32 = 8, TILE_W32x64 = 9, TILE_COUNT = 10 };
 inline int gemm_tile_rows(int t) { const int r[] = {64, 32, 64, 128, 128, 64, 128, 16, 32, 32}; return r[t]; }
 inline int gemm_tile_cols(int t) { const int c[] = {64, 64, 128, 64, 32, 96, 32, 32, 32, 64}; return c[t]; }
+inline bool gemm_tile_direct(int t) { return t == TILE_CONV3; }
 inline bool gemm_tile_wave(int t) { return t == TILE_W16x32 || t == TILE_W32x32 || t == TILE_W32x64; }
 // K and N of a packed B are padded to these.
 constexpr uint32_t PACK_K = 32, PACK_N = 128;
