@@ -763,13 +763,19 @@ bl_binding resolve(const bl_spec &s, uint32_t b, const bl_binding_set &set) {
     return bd;
 }
 
+// Whether launch L's output lies apart from the `bytes` at p: a kernel that
+// writes L's output in L's place may then read them throughout.
+bool apart(const Launch &L, const void *p, uint64_t bytes) {
+    return (const char *)p >= L.out_hi || (const char *)p + bytes <= L.out_lo;
+}
+
 // The class-token prepend fused into the patch embedding that makes its rows
 // (the embeddings' x = [token; patches] + pos): a prepend Q (whole) whose rows
 // are an internal tensor written by nothing but the patch embedding P just
 // before it (whole, no epilogue, not split) and read by nothing but Q. P then
 // writes x's rows 1 .. m itself through Q's epilogue (its added tensors read
 // one row on), its first row band also writes x's first row from the token,
-// and Q launches nothing. Q's epilogue steps must not depend on where a row
+// and Q launches nothing; x lies apart from what P reads, the image and the bias. Q's epilogue steps must not depend on where a row
 // lies: adds of x-shaped tensors, scales, activations, channel scales over a
 // divisor of the row.
 void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32_t *internal, uint32_t n_internal) {
@@ -800,7 +806,8 @@ void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint3
             ok = P.family == Family::GEMM && Q.family == Family::ELEMENT && Q.element == PerElement::PREPEND &&
                  g.load == 2 && g.ksplit <= 1 && !g.flash_ops && !g.c_planes && g.epi_mode == 0 && g.row0 == 0 &&
                  g.row1 == g.m && g.n == Q.el.channels && Q.el.start == 0 &&
-                 Q.el.end == (uint64_t)(g.m + 1) * g.n && P.out_lo == (const char *)Q.el.b && P.f16 == Q.f16;
+                 Q.el.end == (uint64_t)(g.m + 1) * g.n && P.out_lo == (const char *)Q.el.b && P.f16 == Q.f16 &&
+                 apart(Q, g.a, (uint64_t)g.m * g.k * (P.f16 ? 2 : 4)) && (!g.bias || apart(Q, g.bias, g.n * (P.f16 ? 2ull : 4ull)));
             for (int k = 0; k < Q.el.epi.n && ok; k++) {
                 const int kind = Q.el.epi.kind[k];
                 ok = kind == BL_EPI_ADD || kind == BL_EPI_RELU || kind == BL_EPI_GELU || kind == BL_EPI_GELU_ERF ||
@@ -829,12 +836,6 @@ void plan_prepends(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint3
         ks->kernels[qi].label += " > fused into " + std::to_string(pi);
         ks->kernels[pi].label += " < prepend " + std::to_string(qi);
     }
-}
-
-// Whether launch L's output lies apart from the `bytes` at p: a kernel that
-// writes L's output in L's place may then read them throughout.
-bool apart(const Launch &L, const void *p, uint64_t bytes) {
-    return (const char *)p >= L.out_hi || (const char *)p + bytes <= L.out_lo;
 }
 
 // An internal tensor's uses: its one writer and one reader among the kernels

@@ -296,3 +296,23 @@ def test_weights_that_a_kernel_writes_are_packed_again_in_every_set(ctx, product
                 net.kernels.encode_all(s)
                 ctx.synchronize()
                 compare(net.read(101, s), want(np.maximum(w, 0)), math, f"set {s}, weights {seed}: {net.labels}")
+
+
+@pytest.mark.parametrize("math", MATHS, indirect=True)
+def test_tokens_over_the_image_their_patches_come_from(ctx, math):
+    """The plan lays the tokens over an image whose last reader is the patch
+    embedding: the class-token prepend keeps a launch of its own."""
+    grid, p, c, d = 5, 14, 3, 64
+    image, rows = (grid * p) ** 2 * c, grid * grid
+    arrays = [stored(math, a) for a in (oracle.uniform(111, image, 0.0, 1.0), oracle.fan_in_weights(112, p * p * c * d, p * p * c),
+                                        oracle.uniform(113, d, -0.1, 0.1), oracle.uniform(114, d, -1.0, 1.0))]
+    ops = [(ir.op(ir.OP_RELU, [0], [image]), ir.ACTIVATION), (ir.op(ir.OP_PATCH_EMBED, [100, 1, 2], [grid, grid, p, c, d]), ir.ACTIVATION),
+           (ir.op(ir.OP_PREPEND_TOKEN, [3, 101], [rows, d]), ir.ACTIVATION), (ir.op(ir.OP_TOKENS_TO_MAP, [102], [grid, grid, d]), ir.OUTPUT)]
+    with Net(ctx, [(ir.INPUT, image)] + [(ir.WEIGHT, a.size) for a in arrays[1:]], ops, math) as net:
+        assert net.overlap(100, 102), net.labels
+        assert not any("prepend" in lab and "fused" in lab or "< prepend" in lab for lab in net.labels), net.labels
+        for i, a in enumerate(arrays):
+            net.write(i, a)
+        net.kernels.encode_all()
+        ctx.synchronize()
+        compare(net.read(103), oracle.patch_embed(arrays[0], arrays[1], arrays[2], grid, grid, p, c, d), math, f"{net.labels}")
