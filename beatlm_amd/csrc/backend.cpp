@@ -1110,8 +1110,9 @@ void plan_folds(bl_kernels *ks, const bl_spec *specs, uint32_t n, const bl_bindi
             }
             const bl_binding xb = resolve(ls, ls.reads[0], sets[si]);
             const char *x_lo = (const char *)Ln.ln.x, *x_hi = x_lo + xb.size;
-            // Nothing writes x between the LayerNorm and its reader.
-            for (uint32_t j = li + 1; j < (uint32_t)gi && ok; j++)
+            // Nothing writes x between the LayerNorm and its reader, nor, in f16,
+            // does the reader itself, which there reads x and no copy of it.
+            for (uint32_t j = li + 1; j < (uint32_t)gi + (G.math == Math::F16 ? 1 : 0) && ok; j++)
                 if (overlaps(ks->kernels[j].per_set[si], x_lo, x_hi)) ok = false;
             // x's last writer before the LayerNorm, a product writing exactly x.
             int p = -1;

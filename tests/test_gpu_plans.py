@@ -316,3 +316,23 @@ def test_tokens_over_the_image_their_patches_come_from(ctx, math):
         net.kernels.encode_all()
         ctx.synchronize()
         compare(net.read(103), oracle.patch_embed(arrays[0], arrays[1], arrays[2], grid, grid, p, c, d), math, f"{net.labels}")
+
+
+@pytest.mark.parametrize("t,m", [(40, 192), (700, 384)])
+def test_a_product_over_the_input_of_its_folded_layernorm(ctx, t, m):
+    """x -> LayerNorm -> product, x used no further: the plan lays the product
+    over x, which an f16 product with the LayerNorm folded in would still read."""
+    d = 128
+    arrays = [stored("f16", a) for a in (oracle.uniform(121, t * d, -1.0, 1.0), oracle.fan_in_weights(122, d * d, d), oracle.uniform(123, d, 0.8, 1.2),
+                                         oracle.uniform(124, d, -0.1, 0.1), oracle.fan_in_weights(125, d * m, d))]
+    ops = [(ir.op(ir.OP_MATMUL, [0, 1, ir.NONE], [t, d, d]), ir.ACTIVATION), (ir.op(ir.OP_LAYER_NORM, [100, 2, 3], [t, d], EPS), ir.ACTIVATION),
+           (ir.op(ir.OP_MATMUL, [101, 4, ir.NONE], [t, d, m]), ir.ACTIVATION), (ir.op(ir.OP_RESIZE_BILINEAR, [102], [1, t, 1, t, m]), ir.OUTPUT)]
+    with Net(ctx, [(ir.INPUT, t * d)] + [(ir.WEIGHT, a.size) for a in arrays[1:]], ops, "f16") as net:
+        assert net.overlap(100, 102), net.labels
+        assert not any("layernorm 1" in lab for lab in net.labels), net.labels
+        for i, a in enumerate(arrays):
+            net.write(i, a)
+        net.kernels.encode_all()
+        ctx.synchronize()
+        n = oracle.layernorm(oracle.matmul(arrays[0], arrays[1], None, t, d, d), arrays[2], arrays[3], t, d, EPS)
+        compare(net.read(103), oracle.matmul(n, arrays[4], None, t, d, m), "f16", f"{net.labels}")
