@@ -369,9 +369,10 @@ struct Launch {
     // statistics from x when the producer has not written them since x changed.
     int fold = -1;
     int fold_role = 0;
-    // Launches nothing: a class-token prepend fused into the patch embedding
-    // before it, or a token-to-map into the LayerNorm before it, which write
-    // its output.
+    // Launches nothing, its neighbour doing its work: a class-token prepend
+    // (the patch embedding before it), a token-to-map (the LayerNorm before
+    // it), a resampling (the product after it), a one-column product (the
+    // convolution before it).
     bool fused = false;
 };
 enum FoldRole : int { FOLD_NONE = 0, FOLD_LAYER_NORM = 1, FOLD_CONSUMER = 2, FOLD_PRODUCER = 3 };
@@ -428,9 +429,17 @@ struct Fold {
     std::vector<LnStatsArgs> stats;
 };
 
+std::string math_name(Math m) { return m == Math::F32 ? "mfma-f32" : m == Math::F16 ? "mfma-f16" : "mfma-bf16x3"; }
+
 std::string flash_small_name(Math m, uint32_t blocks) {
-    return std::string(m == Math::F32 ? "mfma-f32" : m == Math::F16 ? "mfma-f16" : "mfma-bf16x3") + " 16x16 queries=" +
-           std::to_string(16 * blocks) + " keys over waves";
+    return math_name(m) + " 16x16 queries=" + std::to_string(16 * blocks) + " keys over waves";
+}
+
+// Another variant in a label, between its " @ " and what the kernel gives
+// (" > ...") or takes (" < ...").
+void set_variant(std::string &label, const std::string &variant) {
+    const size_t at = label.find(" @ ") + 3, end = std::min({label.find(" <", at), label.find(" >", at), label.size()});
+    label.replace(at, end - at, variant);
 }
 
 const char *main_name(uint32_t m) {
@@ -1002,6 +1011,7 @@ void plan_resizes(bl_kernels *ks, const bl_spec *specs, uint32_t n, const uint32
             Q.out_lo = Q.out_hi = nullptr;
         }
         ks->kernels[qi].label += " > fused into " + std::to_string(pi);
+        set_variant(ks->kernels[pi].label, math_name(ks->kernels[pi].per_set[0].math) + " rows");
         ks->kernels[pi].label += " < resize " + std::to_string(qi);
     }
 }
@@ -1300,11 +1310,7 @@ void plan_waves(bl_kernels *ks, uint32_t compute_units) {
             L.tile = tile;
             L.gemm.ksplit = L.gemm.kgroups = L.gemm.kslices = 1;
         }
-        const Launch &L = k.per_set[0];
-        const size_t at = k.label.find(" @ "), end = k.label.find(" <", at), end2 = k.label.find(" >", at);
-        const std::string variant = std::string(" @ ") + (L.math == Math::F16 ? "mfma-f16" : L.math == Math::F32 ? "mfma-f32" : "mfma-bf16x3") +
-                                    " wave " + std::to_string(gemm_tile_rows(tile)) + "x" + std::to_string(gemm_tile_cols(tile));
-        k.label.replace(at, std::min(std::min(end, end2), k.label.size()) - at, variant);
+        set_variant(k.label, math_name(k.per_set[0].math) + " wave " + std::to_string(gemm_tile_rows(tile)) + "x" + std::to_string(gemm_tile_cols(tile)));
     }
 }
 
@@ -2160,10 +2166,7 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                 F.fl.prepped = 1;
                 if (const uint32_t small = plan_flash(F.math, F.fl.tokens, F.fl.heads, F.fl.row0, F.fl.row1, ctx->compute_units).small) {
                     F.fl.small = small;
-                    if (si == 0) {
-                        std::string &label = ks->kernels[ki].label;
-                        label.replace(label.find(" @ ") + 3, std::string::npos, flash_small_name(F.math, small));
-                    }
+                    if (si == 0) set_variant(ks->kernels[ki].label, flash_small_name(F.math, small));
                 }
                 F.kv_producers.assign(producers.begin(), producers.end());
                 std::sort(F.kv_producers.begin(), F.kv_producers.end());

@@ -132,6 +132,9 @@ struct DotArgs {
 
 hipError_t launch_gemm_reduce(const GemmArgs &a, bool f16, hipStream_t s);
 
+// K and N of a packed B are padded to these.
+constexpr uint32_t PACK_K = 32, PACK_N = 128;
+
 // B [k][n] -> the GEMM's packed operand (transposed, padded, converted).
 struct PackArgs {
     const void *src;
@@ -280,9 +283,10 @@ struct PointArgs {
 };
 // Vectors of 8 in and out, k of at most three 32-wide slices, 32-bit rows.
 __host__ inline bool point_fits(const PointArgs &a) {
-    return a.k % 8 == 0 && a.k >= 8 && a.k <= 96 && a.n % 8 == 0 && a.n >= 8 && a.n <= (1u << 16) && a.rows > 0 &&
-           a.rows < (1u << 30) && a.k_pad % 32 == 0 && a.k_pad >= a.k && a.n_pad % 128 == 0 && a.n_pad >= a.n && (a.f ? a.cout % 8 == 0 && a.f < 256 && a.n == a.f * a.f * a.cout && !a.ih : a.ih > 0) &&
-           (uint64_t)a.rows * (a.f ? a.f * a.f : 1) < (1ull << 31);
+    if (a.k % 8 != 0 || a.k < 8 || a.k > 96 || a.n % 8 != 0 || a.n < 8 || a.n > (1u << 16) || a.rows == 0 || a.rows >= (1u << 30)) return false;
+    if (a.k_pad % PACK_K != 0 || a.k_pad < a.k || a.n_pad % PACK_N != 0 || a.n_pad < a.n) return false;
+    if (!a.f) return a.ih > 0;
+    return a.f < 256 && !a.ih && a.cout % 8 == 0 && a.n == a.f * a.f * a.cout && (uint64_t)a.rows * a.f * a.f < (1ull << 31);
 }
 constexpr uint32_t POINT_GROUPS = 1024;
 hipError_t launch_point(const PointArgs &a, Math m, hipStream_t s);
@@ -422,8 +426,6 @@ inline int gemm_tile_rows(int t) { const int r[] = {64, 32, 64, 128, 128, 64, 12
 inline int gemm_tile_cols(int t) { const int c[] = {64, 64, 128, 64, 32, 96, 32, 32, 32, 64}; return c[t]; }
 inline bool gemm_tile_direct(int t) { return t == TILE_CONV3; }
 inline bool gemm_tile_wave(int t) { return t == TILE_W16x32 || t == TILE_W32x32 || t == TILE_W32x64; }
-// K and N of a packed B are padded to these.
-constexpr uint32_t PACK_K = 32, PACK_N = 128;
 
 constexpr uint32_t FLASH_HEAD_DIM = 64;
 

@@ -297,9 +297,11 @@ const char *bl_kernels_label(const bl_kernels *kernels, uint32_t kernel);
  * projections again instead, from x as it is, which in program order is the
  * x they read before. Kernels of bl_kernels_create_internal whose work
  * another kernel does launch nothing: a LayerNorm folded into the product
- * that reads it, and a class-token prepend fused into the patch embedding
- * before it (which writes the prepend's output; the internal patches tensor
- * between them is never written). */
+ * that reads it; a class-token prepend, a token-to-map or a one-column product
+ * fused into the patch embedding, LayerNorm or 3x3 convolution before it
+ * (which writes its output when it runs); and a resampling blended into the
+ * product after it (which reads the resampling's input). The internal tensor
+ * between the two is never written. */
 int bl_kernels_encode(bl_kernels *kernels, uint32_t kernel, uint32_t set,
                       bl_timer *timer, uint32_t tag);
 /* Launches kernels [first, first + count) in order with binding set `set`.

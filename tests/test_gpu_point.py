@@ -80,7 +80,7 @@ def test_a_resampling_blended_into_its_product_matches_the_oracle(ctx, ih, iw, o
         y = oracle.resize_bilinear(oracle.conv3x3(x, wc, None, ih, iw, c, c, 1), ih, iw, oh, ow, c)
         return np.maximum(oracle.matmul(y, w, b, oh * ow, c, n), 0)
 
-    check(ctx, arrays, ops, want, math, ["< resize 1", "fused into 2"])
+    check(ctx, arrays, ops, want, math, ["rows < resize 1", "fused into 2"])
 
 
 @pytest.mark.parametrize("h,w,cin", [(130, 255, 32), (67, 513, 40)])
