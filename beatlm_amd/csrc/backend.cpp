@@ -1375,13 +1375,13 @@ namespace {
 
 // One item of the backend's workspace: its bytes, the kernels from its first
 // writer to its last reader (inclusive), its binding set (-1: any), its
-// offset once placed, and whether it shares bytes with no other item.
+// offset once placed, and whether it is a moved tensor.
 struct WsItem {
     uint64_t size;
     uint32_t first, last;
     int set;
     uint64_t at;
-    bool alone = false;
+    bool moved = false;
 };
 
 // Places the items as the memory plan places tensors in an arena
@@ -1390,15 +1390,16 @@ struct WsItem {
 // with. Items of two different binding sets are taken to be live together
 // (a frame loop may interleave the sets' ranges); otherwise two items are
 // live together when their kernel intervals overlap. What shares bytes can be
-// made again (a fold's statistics) or lives for one launch (partial sums); an
-// item that cannot (a moved tensor) is live with every other. Returns the
-// bytes the placement spans.
+// made again (a fold's statistics) or lives for one launch (partial sums). A
+// moved tensor cannot be: it is live with all of those, and shares bytes with
+// moved tensors of its own set alone, as the plan's tensors do in program
+// order. Returns the bytes the placement spans.
 uint64_t place_workspace(std::vector<WsItem> &items) {
     std::vector<size_t> order(items.size());
     for (size_t i = 0; i < order.size(); i++) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return items[a].size > items[b].size; });
     auto together = [&](const WsItem &a, const WsItem &b) {
-        if (a.alone || b.alone || (a.set >= 0 && b.set >= 0 && a.set != b.set)) return true;
+        if (a.moved != b.moved || (a.set >= 0 && b.set >= 0 && a.set != b.set)) return true;
         return a.first <= b.last && b.first <= a.last;
     };
     std::vector<size_t> placed;

@@ -330,7 +330,7 @@ uint64_t bl_kernels_packs_made(const bl_kernels *kernels);
  * planes, and activations moved out of the arenas (a resampling's input that
  * the plan lays under the product which blends it), placed by lifetime as the
  * plan places tensors in an arena (items of disjoint kernel spans share bytes,
- * moved activations with none). No counterpart in the reference, whose
+ * moved activations only with each other). No counterpart in the reference, whose
  * kernels hold no memory of their own; with the arenas' one allocation, a
  * program's device memory is these two allocations. */
 uint64_t bl_kernels_workspace_bytes(const bl_kernels *kernels);
