@@ -2300,7 +2300,8 @@ static hipError_t refresh_pack(bl_kernels *k, const Launch &L, hipStream_t s) {
     return e;
 }
 
-static hipError_t launch(const Launch &L, hipStream_t s) {
+// own_prep: a flash kernel makes K and Vt itself (track_kv).
+static hipError_t launch(const Launch &L, hipStream_t s, bool own_prep = false) {
     if (L.fused) return hipSuccess;  // the kernel beside it does its work
     if (L.point) {
         if (L.gemm.flash_ops) return hipErrorInvalidValue;  // it writes no K or Vt
@@ -2317,7 +2318,12 @@ static hipError_t launch(const Launch &L, hipStream_t s) {
     }
     case Family::GATHER: return launch_gather(L.ga, L.gather, L.f16, s);
     case Family::SOFTMAX: return launch_softmax(L.sm, L.f16, s);
-    case Family::FLASH: return launch_flash(L.fl, L.math, s);
+    case Family::FLASH: {
+        if (!own_prep) return launch_flash(L.fl, L.math, s);
+        FlashArgs fl = L.fl;
+        fl.prepped = 0;
+        return launch_flash(fl, L.math, s);
+    }
     case Family::ELEMENT: return launch_element(L.el, L.element, L.f16, s);
     case Family::DPT: return launch_dpt(L.dp, L.dpt, L.f16, s);
     case Family::GEMV: return launch_gemv(L.gv, L.f16, s);
@@ -2325,13 +2331,6 @@ static hipError_t launch(const Launch &L, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
-// Kernel `i`'s launch `L` as the attention scratch's state `kv` requires it,
-// and that state after it. A flash kernel whose K and Vt its projections
-// write (fl.prepped) reads them from the scratch; when the scratch does not
-// hold them (the flash kernel encoded alone, qkv written since by the host
-// or another kernel, or another flash kernel's operands in between) it runs
-// its own prep instead, which makes them from all of qkv (a kv_rerun flash
-// kernel has its projections run again first: run_one).
 static bool kv_held(const Launch &L, const KvState &kv) {
     if (kv.qkv != L.fl.qkv) return false;
     if (kv.whole) return true;
@@ -2340,25 +2339,28 @@ static bool kv_held(const Launch &L, const KvState &kv) {
     return true;
 }
 
-static Launch with_kv(const Launch &L, uint32_t i, KvState &kv) {
-    Launch run = L;
+// The attention scratch's state `kv` after kernel `i`'s launch `L`, and
+// whether L has to make K and Vt itself first. A flash kernel whose K and Vt
+// its projections write (fl.prepped) reads them from the scratch; when the
+// scratch does not hold them (the flash kernel encoded alone, qkv written
+// since by the host or another kernel, or another flash kernel's operands in
+// between) it runs its own prep instead, which makes them from all of qkv (a
+// kv_rerun flash kernel has its projections run again first: run_one). L is
+// not copied: a launch is some kilobytes, and a slice is bound by its encoding.
+static bool track_kv(const Launch &L, uint32_t i, KvState &kv) {
     if (L.family == Family::FLASH && L.fl.prepped) {
-        if (!kv_held(L, kv)) {
-            run.fl.prepped = 0;
-            kv = KvState{};
-            kv.qkv = L.fl.qkv;
-            kv.lo = (const char *)L.fl.qkv;
-            kv.hi = kv.lo + (uint64_t)3 * L.fl.tokens * L.fl.heads * FLASH_HEAD_DIM * (L.math == Math::F16 ? 2 : 4);
-            kv.whole = true;
-        }
-        return run;
+        if (kv_held(L, kv)) return false;
+        kv = KvState{};
+        kv.qkv = L.fl.qkv;
+        kv.lo = (const char *)L.fl.qkv;
+        kv.hi = kv.lo + (uint64_t)3 * L.fl.tokens * L.fl.heads * FLASH_HEAD_DIM * (L.math == Math::F16 ? 2 : 4);
+        kv.whole = true;
+        return true;
     }
     if (L.family == Family::FLASH) {
         // A flash kernel's own prep overwrites the scratch's operands.
         if (kv.qkv != L.fl.qkv) kv = KvState{};
-        return run;
-    }
-    if (L.family == Family::GEMM && L.gemm.flash_ops) {
+    } else if (L.family == Family::GEMM && L.gemm.flash_ops) {
         if (kv.qkv != L.gemm.c) {
             kv = KvState{};
             kv.qkv = L.gemm.c;
@@ -2366,10 +2368,10 @@ static Launch with_kv(const Launch &L, uint32_t i, KvState &kv) {
             kv.hi = kv.lo + (uint64_t)L.gemm.m * L.gemm.n * (L.math == Math::F16 ? 2 : 4);
         }
         kv.done.push_back(i);
-        return run;
+    } else if (kv.qkv && L.out_lo < kv.hi && kv.lo < L.out_hi) {
+        kv = KvState{};
     }
-    if (kv.qkv && L.out_lo < kv.hi && kv.lo < L.out_hi) kv = KvState{};
-    return run;
+    return false;
 }
 
 static void stale(FoldState &fs, const std::vector<uint32_t> &entries) {
@@ -2409,7 +2411,7 @@ static hipError_t run_one(bl_kernels *k, uint32_t i, uint32_t set, hipStream_t s
         }
         if (!kv_held(L, kv)) return hipErrorInvalidValue;
     }
-    const hipError_t e = launch(with_kv(L, i, kv), s);
+    const hipError_t e = launch(L, s, track_kv(L, i, kv));
     if (e != hipSuccess) return e;
     for (size_t f = 0; f < k->folds.size(); f++) {
         const Fold &fo = k->folds[f];
