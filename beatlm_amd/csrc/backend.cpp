@@ -1440,9 +1440,20 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     ks->ctx = ctx;
     ks->arenas = arenas;
     ks->sets = n_sets;
-    uint64_t scratch_bytes = 0;
-    uint64_t flash_counter_bytes = 0;  // the largest in-kernel merge's arrival counters
-    std::vector<std::pair<size_t, size_t>> flash_users;  // (kernel, set) whose FlashArgs need scratch
+    // The attention scratch: each shape's operands, the largest partial results
+    // and in-kernel merge's arrival counters, and the (kernel, set)s that use it.
+    struct FlashShape {
+        Math math;
+        uint32_t tokens, heads;
+        uint64_t at;
+    };
+    std::vector<FlashShape> flash_shapes;
+    uint64_t flash_operand_bytes = 0, flash_partial_bytes = 0, flash_counter_bytes = 0;
+    std::vector<std::pair<size_t, size_t>> flash_users;
+    auto shape_of_flash = [&](const Launch &L) {
+        return std::find_if(flash_shapes.begin(), flash_shapes.end(),
+                            [&](const FlashShape &s) { return s.math == L.math && s.tokens == L.fl.tokens && s.heads == L.fl.heads; });
+    };
     std::vector<std::pair<size_t, size_t>> split_users;  // (kernel, set) of split-k GEMMs
 
     auto bad = [&](int code, const char *fmt, auto... args) {
@@ -1962,7 +1973,11 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
                 // entry point's bit for bit.
                 L.fl.small = fmath == Math::F32 || getenv("BL_FLASH_SMALL") ? fp.small : 0;
                 L.fl.merge_inline = fp.merge && fp.counters && !getenv("BL_FLASH_MERGE_LAUNCH");
-                scratch_bytes = std::max(scratch_bytes, fp.scratch_bytes);
+                if (shape_of_flash(L) == flash_shapes.end()) {
+                    flash_shapes.push_back({L.math, L.fl.tokens, L.fl.heads, flash_operand_bytes});
+                    flash_operand_bytes += (fp.operand_bytes + 255) / 256 * 256;
+                }
+                flash_partial_bytes = std::max(flash_partial_bytes, fp.scratch_bytes - fp.operand_bytes);
                 flash_counter_bytes = std::max(flash_counter_bytes, fp.counter_bytes);
                 flash_users.push_back({ki, si});
                 variant = L.fl.small ? flash_small_name(fmath, fp.small)
@@ -2060,11 +2075,11 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     if (pack_total) items.push_back({pack_total, 0, whole, -1, 0});
     // The attention scratch: the in-kernel merge's arrival counters in front
     // (every flash kernel's at the same bytes, zero between launches), then
-    // the largest flash kernel's operands and partial results.
+    // each shape's operands, then the largest partial results.
     const uint64_t counter_bytes = align256(flash_counter_bytes);
-    if (scratch_bytes) scratch_bytes = counter_bytes + align256(scratch_bytes);
+    const uint64_t scratch_bytes = flash_users.empty() ? 0 : align256(counter_bytes + flash_operand_bytes + flash_partial_bytes);
     const size_t scratch_item = items.size();
-    if (scratch_bytes) items.push_back({align256(scratch_bytes), 0, whole, -1, 0});
+    if (scratch_bytes) items.push_back({scratch_bytes, 0, whole, -1, 0});
     // Each split-k GEMM's partial sums: the largest over its binding sets,
     // written and read within its own launch.
     std::map<size_t, size_t> partial_item;  // kernel -> item
@@ -2129,12 +2144,16 @@ extern "C" int bl_kernels_create_internal(bl_ctx *ctx, bl_arenas *arenas, const 
     if (scratch_bytes) {
         ks->scratch = ks->workspace + items[scratch_item].at;
         // Kernels run one after another on the stream, so every flash kernel
-        // uses the same scratch: operands, then partial outputs and statistics.
-        for (auto [ki, si] : flash_users)
-            bind_flash_scratch(ks->kernels[ki].per_set[si].fl, ks->kernels[ki].per_set[si].math, ks->scratch, counter_bytes);
+        // uses the same partial results, and those of one shape the same operands.
+        char *operands = (char *)ks->scratch + counter_bytes;
+        for (auto [ki, si] : flash_users) {
+            Launch &L = ks->kernels[ki].per_set[si];
+            bind_flash_scratch(L.fl, L.math, ks->scratch, operands + shape_of_flash(L)->at, operands + flash_operand_bytes);
+        }
         // Zeroed once: the operands' padding keys (past the last token) are
-        // never written by a fused QKV projection and must stay finite, and the
-        // merge's arrival counters start at zero (each launch leaves them so).
+        // never written by a fused QKV projection, nor by another shape's
+        // kernels, and must stay finite; and the merge's arrival counters
+        // start at zero (each launch leaves them so).
         if (hipMemset(ks->scratch, 0, scratch_bytes) != hipSuccess)
             return bad(BL_ERR_HIP, "clearing %llu bytes of attention scratch", (unsigned long long)scratch_bytes);
         // A flash kernel (f16 or bf16x3) whose qkv comes straight from QKV

@@ -1416,7 +1416,8 @@ FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uin
         p.counters = p.merge ? pairs : 0;
         p.counter_bytes = (uint64_t)p.counters * COUNTER_STRIDE * sizeof(uint32_t);
     }
-    p.scratch_bytes = operand_bytes(m, heads, t_pad) + extra;
+    p.operand_bytes = operand_bytes(m, heads, t_pad);
+    p.scratch_bytes = p.operand_bytes + extra;
     p.small = small_blocks(p, m, tokens, heads, rows, compute_units);
     return p;
 }
@@ -1466,13 +1467,11 @@ int flash_plan_check(uint32_t tokens, uint32_t heads, uint32_t compute_units, bo
     return total == p.units ? BL_OK : BL_ERR_KERNEL;
 }
 
-void bind_flash_scratch(FlashArgs &a, Math m, void *base, uint64_t counter_bytes) {
-    const uint64_t ops = operand_bytes(m, a.heads, a.t_pad);
-    a.counters = (uint32_t *)base;
-    char *b = (char *)base + counter_bytes;
-    a.kp = b;
-    a.vt = b + ops / 2;
-    a.partial = (float *)(b + ops);
+void bind_flash_scratch(FlashArgs &a, Math m, void *counters, void *operands, void *partials) {
+    a.counters = (uint32_t *)counters;
+    a.kp = operands;
+    a.vt = (char *)operands + operand_bytes(m, a.heads, a.t_pad) / 2;
+    a.partial = (float *)partials;
     if (m == Math::F32) {
         a.stats = a.partial + (uint64_t)a.splits * a.tokens * a.heads * HD;
     } else {

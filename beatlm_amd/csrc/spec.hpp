@@ -236,7 +236,7 @@ struct FlashPlan {
     // in-kernel merge (`counters` words, one per (head, query tile) pair) are
     // not counted: they sit in a region of their own in front, shared by every
     // flash kernel of the scratch and zero between launches.
-    uint64_t scratch_bytes = 0;
+    uint64_t scratch_bytes = 0, operand_bytes = 0;  // operand_bytes: the operands' share
     uint32_t counters = 0;
     uint64_t counter_bytes = 0;  // the counters' bytes (each on a line of its own)
     // False when the shape's unit runs would overflow the kernels' 32-bit
@@ -354,10 +354,10 @@ hipError_t launch_gather(const GatherArgs &a, Gather g, bool f16, hipStream_t s)
 hipError_t launch_softmax(const SoftmaxArgs &a, bool f16, hipStream_t s);
 hipError_t launch_flash(const FlashArgs &a, Math m, hipStream_t s);
 FlashPlan plan_flash(Math m, uint32_t tokens, uint32_t heads, uint32_t row0, uint32_t row1, uint32_t compute_units);
-// Points a planned FlashArgs at its scratch: the counter region of
-// counter_bytes (at least the plan's counter_bytes, zero) at `base`, then
-// plan.scratch_bytes of operands and partial results.
-void bind_flash_scratch(FlashArgs &a, Math m, void *base, uint64_t counter_bytes);
+// Points a planned FlashArgs at its scratch: the arrival counters (zero, the
+// plan's counter_bytes at least), its operands (plan.operand_bytes) and its
+// partial results (the rest of plan.scratch_bytes).
+void bind_flash_scratch(FlashArgs &a, Math m, void *counters, void *operands, void *partials);
 hipError_t launch_element(const ElementArgs &a, PerElement p, bool f16, hipStream_t s);
 hipError_t launch_spin(uint64_t ticks, uint32_t blocks, hipStream_t s);
 hipError_t launch_dpt(const DptArgs &a, Dpt k, bool f16, hipStream_t s);

@@ -125,7 +125,8 @@ extern "C" int bl_flash_attention_static(bl_ctx *ctx, const void *qkv, void *out
     a.small = m == bl::Math::F32 ? plan.small : 0;  // as bl_kernels_encode without a projection before it
     a.merge_inline = plan.merge && plan.counters;
     a.prepped = 0;  // the prep launch writes K and Vt into the scratch
-    bl::bind_flash_scratch(a, m, base, COUNTER_BYTES);
+    char *operands = (char *)base + COUNTER_BYTES;
+    bl::bind_flash_scratch(a, m, base, operands, operands + plan.operand_bytes);
     e = bl::launch_flash(a, m, bl_stream_of(ctx));
     return e == hipSuccess ? BL_OK : bl_fail(ctx, BL_ERR_HIP, hipGetErrorString(e));
 }

@@ -336,3 +336,31 @@ def test_a_product_over_the_input_of_its_folded_layernorm(ctx, t, m):
         ctx.synchronize()
         n = oracle.layernorm(oracle.matmul(arrays[0], arrays[1], None, t, d, d), arrays[2], arrays[3], t, d, EPS)
         compare(net.read(103), oracle.matmul(n, arrays[4], None, t, d, m), "f16", f"{net.labels}")
+
+
+@pytest.mark.parametrize("t1,t2", [(300, 705), (257, 641), (900, 1985)])
+@pytest.mark.parametrize("math", ["bf16x3", "f16"], indirect=True)
+def test_attentions_of_two_sizes_share_their_scratch(ctx, monkeypatch, t1, t2, math):
+    """The larger attention's keys past its last token lie where the smaller
+    one's partial results would: they must stay finite, whatever ran before."""
+    monkeypatch.setenv("BL_FLASH_SMALL", "0")
+    heads, d = 2, 128
+    arrays, ops = [], []
+    for i, t in enumerate((t1, t2)):
+        arrays += [stored(math, a) for a in (oracle.uniform(131 + i, t * d, -1.0, 1.0), oracle.fan_in_weights(133 + i, 3 * d * d, d),
+                                             oracle.uniform(135 + i, 3 * d, -0.1, 0.1))]
+        b = 100 + 5 * i
+        # The first qkv is an output: the two lie at places of their own.
+        ops += [(ir.op(ir.OP_MATMUL, [3 * i, 3 * i + 1, 3 * i + 2], [t, d, 3 * d]), ir.ACTIVATION if i else ir.OUTPUT),
+                (ir.op(ir.OP_ATTENTION_SCORES, [b], [t, heads, 64]), ir.ACTIVATION), (ir.op(ir.OP_SCALE, [b + 1], [t * heads * t], 0.125), ir.ACTIVATION),
+                (ir.op(ir.OP_SOFTMAX, [b + 2], [t * heads, t]), ir.ACTIVATION),
+                (ir.op(ir.OP_ATTENTION_VALUES, [b + 3, b], [t, heads, 64]), ir.OUTPUT)]
+    with Net(ctx, [(ir.WEIGHT if i % 3 else ir.INPUT, a.size) for i, a in enumerate(arrays)], ops, math) as net:
+        for i, a in enumerate(arrays):
+            net.write(i, a)
+        for _ in range(3):
+            net.kernels.encode_all()
+        ctx.synchronize()
+        for i, t in enumerate((t1, t2)):
+            qkv = stored(math, oracle.matmul(arrays[3 * i], arrays[3 * i + 1], arrays[3 * i + 2], t, d, 3 * d))
+            compare(net.read(104 + 5 * i), oracle.attention(qkv, t, heads, 64, 0.125), math, f"{t} tokens, {net.labels}")
